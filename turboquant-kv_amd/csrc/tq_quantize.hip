@@ -21,6 +21,7 @@
 // rounding helpers are the identity.
 
 #include "tq_common.h"
+#include "tq_q16.h"
 
 namespace tq {
 
@@ -720,83 +721,118 @@ __global__ __launch_bounds__(kThreads) void dequant_kernel(DequantArgs a) {
   }
 }
 
-// ---------------------------------------------------------------- one row per wave (few rows)
-// quantize_kernel<false>'s arithmetic, bit for bit, for bf16/fp16 inputs of d = 64 / 128,
-// with one wave per row (lane j owns output dims j and j + 64): a decode step appends one
-// token per (sequence, KV head) -- a few hundred rows -- which 16-row tiles would spread
-// over a few dozen workgroups, each walking its tile through five barriers.  Here R (its
-// elements rounded to the input type, transposed: Rt[k][j]) sits in LDS; per row the norm
-// (fmaf over the lane's dims, then the wave sum: tile_norms' order), the unit vector
-// (rounded), y_j = sum_k fmaf(u_k, R[j][k]) for k ascending (contract_rows' order), the
-// code (count_below) and the bit planes from ballots (dim j at bit 7 - j % 8 of byte j / 8).
-constexpr int kQrThreads = 256;
-constexpr int64_t kQrMaxRows = 16384;  // above this the tiled kernel is as fast
+// ---------------------------------------------------------------- 16-bit rows, d 64 / 128
+// q16::Quantizer's codes as bit planes: a wave takes 16 rows at a time, the next tile's rows
+// loaded while the current one is worked on.  Lane (row, g) holds the codes of D/4
+// consecutive dims, a share of every plane; the four lane groups exchange shares by
+// permlane swaps so that group p stores plane p of its rows whole (16 or 8 bytes).
+struct Q16Args {
+  const uint16_t* x;  // [n, D]
+  int64_t n;
+  const float* rot;
+  const float* bnd;
+  int bits;
+  uint8_t* packed;    // [n, bits D / 8]
+  void* norms;        // [n], norm_dt
+  int norm_dt;
+};
 
-template <int D>
-__global__ __launch_bounds__(kQrThreads) void quantize_rows_kernel(QuantArgs a) {
-  constexpr int C = D / 64;  // output dims per lane
-  constexpr int BPP = D / 8;
-  __shared__ float rt_s[D][D + 1];  // padded: the transposing writes hit distinct banks
-  __shared__ float u_s[kQrThreads / 64][D];
-  __shared__ float bnd_s[16];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int rdt = a.rdt;
-  const int nlev = 1 << a.bits;
-  if (threadIdx.x < nlev - 1) bnd_s[threadIdx.x] = round_to(a.bnd[threadIdx.x], rdt);
-  for (int e = threadIdx.x; e < D * D; e += kQrThreads) {  // coalesced read of R row j
-    const int j = e / D, k = e - j * D;
-    rt_s[k][j] = round_to(a.rot[e], rdt);
-  }
-  __syncthreads();
-  const float eps = round_to(1e-10f, rdt);
-  const int P = a.bits * BPP;
-  for (int64_t row = (int64_t)blockIdx.x * (kQrThreads / 64) + wave; row < a.n;
-       row += (int64_t)gridDim.x * (kQrThreads / 64)) {
-    float x[C];
+template <int D, bool BF>
+__global__ __launch_bounds__(64 * q16::waves<D>(), 4) void quantize16_kernel(Q16Args a) {
+  using Q = q16::Quantizer<D, BF, true>;
+  __shared__ q16::Lds<D> t;
+  __shared__ q16::WaveLds<D> wl[Q::W];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15;
+  const int nb = (1 << a.bits) - 1;
+  const int64_t step = (int64_t)gridDim.x * Q::W;
+  const int64_t ntiles = (a.n + 15) / 16;
+  int64_t tile = (int64_t)blockIdx.x * Q::W + wave;
+  q16::v4u x[Q::KS];
+  auto load_rows = [&](int64_t tl) {
+    const int64_t row = tl * 16 + c16;
 #pragma unroll
-    for (int c = 0; c < C; ++c) x[c] = load_as_f32(a.x, row * D + lane + 64 * c, a.in_dt);
-    float ss = 0.f;
+    for (int s = 0; s < Q::KS; ++s)
+      x[s] = row < a.n ? *reinterpret_cast<const q16::v4u*>(a.x + row * D + 32 * s + 8 * g) : (q16::v4u){0, 0, 0, 0};
+  };
+  Q::fill(t, a.rot, a.bnd, nb, [&] { if (tile < ntiles) load_rows(tile); });
+  Q q;
+  q.load(t, nb);
+  constexpr int PB = D / 8;  // bytes per plane
+  const bool wide = (reinterpret_cast<uintptr_t>(a.packed) & (PB - 1)) == 0;
+  for (; tile < ntiles; tile += step) {
+    q16::v4u xc[Q::KS];
 #pragma unroll
-    for (int c = 0; c < C; ++c) ss = fmaf(x[c], x[c], ss);
-    ss = wave_sum(ss);
-    const float nrm = round_to(sqrtf(ss), rdt);
-    if (lane == 0) a.norms[row] = nrm;
-    const float den = fmaxf(nrm, eps);
+    for (int s = 0; s < Q::KS; ++s) xc[s] = x[s];
+    if (tile + step < ntiles) load_rows(tile + step);
+    uint32_t code[Q::CT];
+    const float nrm = q.tile(t, wl[wave], nb, xc, code);
+    const int64_t row = tile * 16 + c16;
+    const bool live = row < a.n;
+    if (g == 0 && live) store_from_f32(a.norms, row, nrm, a.norm_dt);
+    uint32_t nib[D / 32];
 #pragma unroll
-    for (int c = 0; c < C; ++c) u_s[wave][lane + 64 * c] = round_to(x[c] / den, rdt);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    float acc[C];
+    for (int i = 0; i < D / 32; ++i) nib[i] = q16::nibbles8(code[2 * i], code[2 * i + 1]);
+    uint8_t* dst = a.packed + row * (int64_t)(a.bits * PB);
+    if constexpr (D == 128) {
+      uint32_t pl[4];
 #pragma unroll
-    for (int c = 0; c < C; ++c) acc[c] = 0.f;
-#pragma unroll 8
-    for (int k = 0; k < D; ++k) {
-      const float uk = u_s[wave][k];
+      for (int p = 0; p < 4; ++p) {
+        pl[p] = 0;
+        if (p < a.bits) {
 #pragma unroll
-      for (int c = 0; c < C; ++c) acc[c] = fmaf(uk, rt_s[k][lane + 64 * c], acc[c]);
-    }
-    uint32_t code[C];
-#pragma unroll
-    for (int c = 0; c < C; ++c) code[c] = (uint32_t)count_below(bnd_s, nlev, round_to(acc[c], rdt));
-    // lane L < P writes byte L of the row: plane L / BPP, dims 8 (L % BPP) .. + 7
-    uint8_t out = 0;
-#pragma unroll
-    for (int pl = 0; pl < 4; ++pl) {
-      if (pl < a.bits) {
-#pragma unroll
-        for (int c = 0; c < C; ++c) {
-          const uint64_t m = __ballot((code[c] >> pl) & 1u);
-          const int b = lane - pl * BPP - 8 * c;  // byte of this plane held in mask c
-          if (b >= 0 && b < 8)
-            out = (uint8_t)(__builtin_bitreverse32((uint32_t)(m >> (8 * b)) & 0xFFu) >> 24);
+          for (int i = 0; i < 4; ++i) pl[p] |= q16::plane8(nib[i], p) << (8 * i);
         }
       }
+      const auto s0 = __builtin_amdgcn_permlane32_swap(pl[0], pl[2], false, false);
+      const auto s1 = __builtin_amdgcn_permlane32_swap(pl[1], pl[3], false, false);
+      const auto s2 = __builtin_amdgcn_permlane16_swap(s0[0], s1[0], false, false);
+      const auto s3 = __builtin_amdgcn_permlane16_swap(s0[1], s1[1], false, false);
+      const uint4 v = make_uint4(s2[0], s2[1], s3[0], s3[1]);  // plane g, words of groups 0..3
+      if (live && g < a.bits) {
+        if (wide) *reinterpret_cast<uint4*>(dst + g * PB) = v;
+        else
+#pragma unroll
+          for (int i = 0; i < 16; ++i)
+            dst[g * PB + i] = (uint8_t)((i < 4 ? v.x : i < 8 ? v.y : i < 12 ? v.z : v.w) >> (8 * (i & 3)));
+      }
+    } else {
+      uint32_t pl[4];  // 16 bits each
+#pragma unroll
+      for (int p = 0; p < 4; ++p)
+        pl[p] = p < a.bits ? q16::plane8(nib[0], p) | q16::plane8(nib[1], p) << 8 : 0u;
+      // groups g and g + 2 pair up: x0 holds planes (0, 1) (lower groups) or (2, 3) of the
+      // lower partner, x1 of the upper one
+      const auto s = __builtin_amdgcn_permlane32_swap(pl[0] | pl[1] << 16, pl[2] | pl[3] << 16, false, false);
+      const uint32_t e0 = __builtin_amdgcn_perm(s[1], s[0], 0x05040100u);  // even plane: partners g, g + 2
+      const uint32_t e1 = __builtin_amdgcn_perm(s[1], s[0], 0x07060302u);  // odd plane
+      const auto w = __builtin_amdgcn_permlane16_swap(e0, e1, false, false);  // groups (0, 2), (1, 3)
+      const uint2 v = make_uint2(__builtin_amdgcn_perm(w[1], w[0], 0x05040100u),
+                                 __builtin_amdgcn_perm(w[1], w[0], 0x07060302u));
+      if (live && g < a.bits) {
+        if (wide) *reinterpret_cast<uint2*>(dst + g * PB) = v;
+        else
+#pragma unroll
+          for (int i = 0; i < 8; ++i) dst[g * PB + i] = (uint8_t)((i < 4 ? v.x : v.y) >> (8 * (i & 3)));
+      }
     }
-    if (lane < P) a.packed[row * P + lane] = out;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();  // u_s is rewritten by the next row
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+}
+
+bool use_q16(const void* x, tq_dtype in_dt, tq_dtype rdt, int d) {
+  return in_dt != TQ_F32 && in_dt == rdt && (d == 64 || d == 128) &&
+         (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
+}
+
+void launch_q16(const Q16Args& a, int d, tq_dtype dt, hipStream_t st) {
+  const int w = d == 128 ? q16::waves<128>() : q16::waves<64>();
+  const int64_t want = (a.n + 16 * w - 1) / (16 * w), cap = (int64_t)device_cu_count() * (d == 128 ? 2 : 4);
+  const dim3 grid((unsigned)(want < cap ? want : cap)), blk(64 * w);
+  if (d == 128) {
+    if (dt == TQ_BF16) hipLaunchKernelGGL((quantize16_kernel<128, true>), grid, blk, 0, st, a);
+    else hipLaunchKernelGGL((quantize16_kernel<128, false>), grid, blk, 0, st, a);
+  } else {
+    if (dt == TQ_BF16) hipLaunchKernelGGL((quantize16_kernel<64, true>), grid, blk, 0, st, a);
+    else hipLaunchKernelGGL((quantize16_kernel<64, false>), grid, blk, 0, st, a);
   }
 }
 
@@ -894,19 +930,30 @@ int tq_rotate_and_quantize(const void* vectors, tq_dtype in_dtype, tq_dtype roun
     TQ_LAUNCH_CHECK("quantize_mfma_kernel<mse>");
     return TQ_OK;
   }
-  if ((d == 64 || d == 128) && in_dtype != TQ_F32 && n <= kQrMaxRows) {  // few rows: a wave each
-    const int64_t waves_per_cu = d == 64 ? 16 : 8;  // LDS: 16 / 64 KB of R per workgroup
-    const int64_t cap = (int64_t)device_cu_count() * waves_per_cu / (kQrThreads / 64);
-    const int64_t want = (n + kQrThreads / 64 - 1) / (kQrThreads / 64);
-    const dim3 grid((unsigned)(want < cap ? want : cap));
-    if (d == 64) hipLaunchKernelGGL(quantize_rows_kernel<64>, grid, dim3(kQrThreads), 0, as_stream(stream), a);
-    else hipLaunchKernelGGL(quantize_rows_kernel<128>, grid, dim3(kQrThreads), 0, as_stream(stream), a);
-    TQ_LAUNCH_CHECK("quantize_rows_kernel");
-    return TQ_OK;
-  }
+  if (use_q16(vectors, in_dtype, round_dtype, d))
+    return tq_quantize_mse_rows(vectors, in_dtype, n, d, rotation, boundaries, bit_width, packed, norms, TQ_F32,
+                                stream);
   hipLaunchKernelGGL(quantize_kernel<false>, dim3(grid_for_tiles(n)), dim3(kThreads), 0,
                      as_stream(stream), a);
   TQ_LAUNCH_CHECK("quantize_kernel<mse>");
+  return TQ_OK;
+}
+
+int tq_quantize_mse_rows(const void* vectors, tq_dtype dtype, int64_t n, int32_t d,
+                         const float* rotation, const float* boundaries, int32_t bit_width,
+                         uint8_t* packed, void* norms, tq_dtype norm_dtype, void* stream) {
+  TQ_REQUIRE(bit_width >= 1 && bit_width <= 4, "bit_width must be 1-4, got %d", bit_width);
+  TQ_REQUIRE(d == 64 || d == 128, "dim must be 64 or 128, got %d", d);
+  TQ_REQUIRE(n >= 0, "n must be >= 0");
+  TQ_REQUIRE(dtype == TQ_BF16 || dtype == TQ_F16, "rows must be bf16 or fp16");
+  TQ_REQUIRE(norm_dtype == dtype || norm_dtype == TQ_F32, "norms are float32 or the rows' type");
+  if (n == 0) return TQ_OK;
+  TQ_REQUIRE(vectors && rotation && boundaries && packed && norms, "null pointer argument");
+  TQ_REQUIRE(use_q16(vectors, dtype, dtype, d), "rows must be 16-byte aligned");
+  launch_q16(Q16Args{static_cast<const uint16_t*>(vectors), n, rotation, boundaries, bit_width, packed, norms,
+                     (int)norm_dtype},
+             d, dtype, as_stream(stream));
+  TQ_LAUNCH_CHECK("quantize16_kernel");
   return TQ_OK;
 }
 
