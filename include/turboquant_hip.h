@@ -315,6 +315,25 @@ int tq_decode_attention_packed(const void* q, tq_dtype q_dtype, int32_t B, int32
                                void* stream);
 
 /*
+ * A decode-layout cache's first T tokens of every (batch row, head) dequantized, followed by
+ * n_new tokens copied as they are: keys / values [batch][heads][T + n_new][d] in out_dtype,
+ * the tensors the reference's cache hands to a model's attention
+ * (hf_integration.py:370-421).  tq_unpack_decode_layout + tq_dequantize_mse (norms first
+ * rounded to out_dtype where they are wider) and the concatenation in one launch.  kpairs /
+ * vtiles / norms as tq_cache_append_dl writes them (4-bit keys, vbits 2-4, d 64 or 128);
+ * key_new / value_new: element (b, h, i, j) at strides[0] b + strides[1] h + strides[2] i + j,
+ * rows 16-byte aligned; null with n_new = 0.
+ */
+int tq_dequantize_cache_dl(const uint8_t* kpairs, const void* knorms, const uint8_t* vtiles,
+                           const void* vnorms, tq_dtype norm_dtype, int64_t batch, int32_t heads,
+                           int32_t d, int64_t t_cap, int64_t T, int32_t vbits,
+                           const float* kcentroids, const float* krotation,
+                           const float* vcentroids, const float* vrotation, const void* key_new,
+                           const int64_t* key_strides, const void* value_new,
+                           const int64_t* value_strides, int64_t n_new, tq_dtype out_dtype,
+                           void* keys, void* values, void* stream);
+
+/*
  * Decode layout: the codes of a packed KV cache with 4-bit keys and 2-, 3- or 4-bit
  * values arranged for the decode kernel, same bytes per token as the bit-plane rows.
  * The reference stores its cache privately (cache.py:81-130), so this arrangement is

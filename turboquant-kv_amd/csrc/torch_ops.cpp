@@ -1197,6 +1197,64 @@ void cache_append_dl(const at::Tensor& key, const at::Tensor& value, at::Tensor&
   }
 }
 
+// The first T tokens of a decode-layout cache dequantized to `out_like`'s dtype, then the new
+// tokens key_new / value_new [B, H, s, d] as they are: (keys, values) [B, H, T + s, d].
+std::tuple<at::Tensor, at::Tensor> dequantize_cache_dl(
+    const at::Tensor& kp, const at::Tensor& kn, const at::Tensor& vp, const at::Tensor& vn, int64_t T,
+    const at::Tensor& kcentroids, const at::Tensor& krotation, const at::Tensor& vcentroids,
+    const at::Tensor& vrotation, at::ScalarType dtype, const c10::optional<at::Tensor>& key_new,
+    const c10::optional<at::Tensor>& value_new) {
+  require_gpu(kp, "kp");
+  c10::DeviceGuard g(kp.device());
+  const auto dev = kp.device();
+  TORCH_CHECK(kp.dim() == 4 && vp.dim() == 4 && kp.is_contiguous() && vp.is_contiguous() &&
+                  kp.scalar_type() == at::kByte && vp.scalar_type() == at::kByte && vp.device() == dev,
+              "kp / vp must be contiguous uint8 decode-layout caches");
+  const int64_t B = kp.size(0), H = kp.size(1), t_cap = kp.size(2), d = kp.size(3) * 2;
+  TORCH_CHECK(d == 64 || d == 128, "head_dim must be 64 or 128");
+  const int64_t vb = vp.size(3) / (8 * d);
+  TORCH_CHECK(vp.size(0) == B && vp.size(1) == H && vp.size(2) * 64 == t_cap && vp.size(3) == 8 * vb * d && vb >= 2 &&
+                  vb <= 4,
+              "vp must be [B, H, t_cap/64, 8 value_bits d]");
+  TORCH_CHECK(kn.device() == dev && vn.device() == dev && kn.is_contiguous() && vn.is_contiguous() &&
+                  kn.numel() == B * H * t_cap && vn.numel() == kn.numel() && kn.scalar_type() == vn.scalar_type() &&
+                  (kn.scalar_type() == at::kFloat || kn.scalar_type() == dtype),
+              "kn / vn must be contiguous [B, H, t_cap], float32 or the output's dtype");
+  TORCH_CHECK(T >= 0 && T <= t_cap, "T past the cache's capacity");
+  auto kc = f32c(kcentroids, dev), vc = f32c(vcentroids, dev);
+  auto Rk = f32c(krotation, dev), Rv = f32c(vrotation, dev);
+  TORCH_CHECK(kc.numel() == 16 && vc.numel() == (1 << vb), "centroids: 16 of the keys, 2^bits of the values");
+  TORCH_CHECK(Rk.numel() == d * d && Rv.numel() == d * d, "rotations must be [d, d]");
+  TORCH_CHECK(key_new.has_value() == value_new.has_value(), "key_new and value_new go together");
+  at::Tensor k1, v1;
+  int64_t s = 0, ks[3] = {0, 0, 0}, vs[3] = {0, 0, 0};
+  if (key_new.has_value()) {
+    TORCH_CHECK(key_new->dim() == 4 && key_new->size(0) == B && key_new->size(1) == H && key_new->size(3) == d &&
+                    value_new->sizes() == key_new->sizes(),
+                "key_new / value_new must be [B, H, s, d]");
+    s = key_new->size(2);
+    const int64_t piece = 16 / (int64_t)at::elementSize(dtype);
+    auto rows = [&](const at::Tensor& t) {  // rows of d elements in 16-byte pieces
+      auto x = t.to(dev, dtype);
+      const bool ok = x.stride(3) == 1 && x.stride(0) % piece == 0 && x.stride(1) % piece == 0 &&
+                      x.stride(2) % piece == 0 && (reinterpret_cast<uintptr_t>(x.data_ptr()) & 15) == 0;
+      return ok ? x : x.clone(at::MemoryFormat::Contiguous);
+    };
+    k1 = rows(*key_new);
+    v1 = rows(*value_new);
+    for (int i = 0; i < 3; ++i) { ks[i] = k1.stride(i); vs[i] = v1.stride(i); }
+  }
+  auto ko = at::empty({B, H, T + s, d}, kp.options().dtype(dtype));
+  auto vo = at::empty({B, H, T + s, d}, kp.options().dtype(dtype));
+  if (B * H * (T + s) == 0) return {ko, vo};
+  check_rc(tq_dequantize_cache_dl(
+      kp.data_ptr<uint8_t>(), kn.data_ptr(), vp.data_ptr<uint8_t>(), vn.data_ptr(), to_tq(kn.scalar_type()), B,
+      (int32_t)H, (int32_t)d, t_cap, T, (int32_t)vb, kc.data_ptr<float>(), Rk.data_ptr<float>(), vc.data_ptr<float>(),
+      Rv.data_ptr<float>(), s ? k1.data_ptr() : nullptr, ks, s ? v1.data_ptr() : nullptr, vs, s, to_tq(dtype),
+      ko.data_ptr(), vo.data_ptr(), cur_stream(kp)));
+  return {ko, vo};
+}
+
 // The exact current token merged into a decode output by log-sum-exp
 // (hf_integration.py:372-390): o [B, Hq, d] and lse [B, Hq] from a *_lse decode op, q
 // [B, Hq, d], k_new / v_new [B, Hkv, d]; returns [B, Hq, d] in q.dtype.
@@ -1324,6 +1382,9 @@ TORCH_LIBRARY(turboquant, m) {
   m.def("cache_append_dl(Tensor key, Tensor value, Tensor(a!) kp, Tensor(b!) kn, Tensor(c!) vp,"
         " Tensor(d!) vn, int pos, Tensor krotation, Tensor kboundaries, Tensor vrotation,"
         " Tensor vboundaries, int kbits, int vbits) -> ()");
+  m.def("dequantize_cache_dl(Tensor kp, Tensor kn, Tensor vp, Tensor vn, int T, Tensor kcentroids,"
+        " Tensor krotation, Tensor vcentroids, Tensor vrotation, ScalarType dtype, Tensor? key_new=None,"
+        " Tensor? value_new=None) -> (Tensor, Tensor)");
   m.def("paged_store_value_tiles(Tensor rows, Tensor norms, Tensor slot_mapping,"
         " Tensor(a!) vtile_pool, Tensor(b!) vnorm_pool) -> ()");
   m.def("decode_attention_paged_dl(Tensor q, Tensor kpairs_pool, Tensor knorm_pool,"
@@ -1372,4 +1433,5 @@ TORCH_LIBRARY_IMPL(turboquant, CUDA, m) {
   m.impl("decode_merge_token", &decode_merge_token);
   m.impl("decode_attention_dl_merged", &decode_attention_dl_merged);
   m.impl("cache_append_dl", &cache_append_dl);
+  m.impl("dequantize_cache_dl", &dequantize_cache_dl);
 }

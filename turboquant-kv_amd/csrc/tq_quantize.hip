@@ -25,6 +25,9 @@
 
 namespace tq {
 
+bool dequant_rows_mfma(const uint8_t* packed, const float* norms, int64_t n, int d, int bits, const float* cen,
+                       const float* rot, int out_dt, void* out, hipStream_t st);  // tq_dequant.hip
+
 std::string& last_error() {
   static thread_local std::string msg;
   return msg;
@@ -1018,6 +1021,10 @@ int tq_dequantize_mse(const uint8_t* packed, const float* norms, int64_t n, int3
   TQ_REQUIRE(valid_dtype(out_dtype), "unknown dtype");
   if (n == 0) return TQ_OK;
   TQ_REQUIRE(packed && norms && centroids && rotation && out, "null pointer argument");
+  if (dequant_rows_mfma(packed, norms, n, d, bit_width, centroids, rotation, (int)out_dtype, out, as_stream(stream))) {
+    TQ_LAUNCH_CHECK("dequant_rows_kernel");
+    return TQ_OK;
+  }
   DequantArgs a{packed, nullptr, nullptr, norms, n, d, bit_width, centroids, rotation, nullptr,
                 out_dtype, out};
   hipLaunchKernelGGL(dequant_kernel<false>, dim3(grid_for_tiles(n)), dim3(kThreads), 0,

@@ -85,6 +85,15 @@ class _Quantizer:
                                             self.d)
 
 
+def _tracked(device, *tensors: torch.Tensor) -> bool:
+    """Whether a derivative of the tensors is wanted (reverse or forward mode), or they are
+    not plain tensors on the device: they then go through torch's own concatenation."""
+    from torch.autograd import forward_ad
+    return (forward_ad._current_level >= 0 or
+            any(type(t) is not torch.Tensor or t.device != device or (t.requires_grad and torch.is_grad_enabled())
+                for t in tensors))
+
+
 class TurboQuantLayer(_HFLayer):
     """Packed KV storage of one transformer layer."""
 
@@ -196,6 +205,8 @@ class TurboQuantLayer(_HFLayer):
         if T == 0:
             z = torch.zeros(B, H, 0, d, dtype=self.dtype, device=self.device)
             return z, z.clone()
+        if self._dl_dequantizes():
+            return self._dequantize_dl(T)
         res = []
         for q, p, n, sg, rs in ((self.kq, self.kp, self.kn, "ks", "kr"),
                                 (self.vq, self.vp, self.vn, "vs", "vr")):
@@ -209,6 +220,13 @@ class TurboQuantLayer(_HFLayer):
                                    dtype=self.dtype)
             res.append(out.view(B, H, T, d).to(self.dtype))
         return res[0], res[1]
+
+    def _dl_dequantizes(self) -> bool:
+        return self.dl and self.dtype in (torch.float32, torch.bfloat16, torch.float16)
+
+    def _dequantize_dl(self, T: int, key_new=None, value_new=None):
+        return _ops().dequantize_cache_dl(self.kp, self.kn, self.vp, self.vn, T, self.kq.cen, self.kq.R,
+                                          self.vq.cen, self.vq.R, self.dtype, key_new, value_new)
 
     def rows(self, values: bool, T: Optional[int] = None) -> torch.Tensor:
         """Bit-plane packed rows [B, H, T, P] of tokens 0..T-1 (reference.py:191-224),
@@ -238,6 +256,11 @@ class TurboQuantLayer(_HFLayer):
         if self.fused_attention:
             self._append(key_states, value_states)
             return _FusedKV(key_states, self, t_hist), value_states
+        if t_hist > 0 and self._dl_dequantizes() and not _tracked(self.kp.device, key_states, value_states):
+            # history and new tokens written into the returned tensors by one kernel
+            out = self._dequantize_dl(t_hist, key_states, value_states)
+            self._append(key_states, value_states)
+            return out
         k_old, v_old = self.dequantized()
         self._append(key_states, value_states)
         return (torch.cat([k_old, key_states.to(self.dtype)], dim=-2),
