@@ -315,6 +315,38 @@ int tq_decode_attention_packed(const void* q, tq_dtype q_dtype, int32_t B, int32
                                void* stream);
 
 /*
+ * n new tokens of every (batch row, head), bf16 / fp16, quantized and written at positions
+ * pos .. pos + n - 1 of a decode-layout cache in one launch: codes and norms equal
+ * tq_rotate_and_quantize (rounding in in_dtype) followed by tq_pack_decode_layout bit for bit
+ * (QuantizedKVCache.append, cache.py:132-207).  key / value: element (b, h, i, j) at
+ * strides[0] b + strides[1] h + strides[2] i + j.  kpairs [batch heads][t_cap][d/2], vtiles
+ * [batch heads][t_cap/64][8 vbits d] (both 16-byte aligned), knorms / vnorms
+ * [batch heads][t_cap] in norm_dtype.  d 64 or 128, vbits 2-4.
+ */
+int tq_cache_append_tokens_dl(const void* key, const int64_t* key_strides, const void* value,
+                              const int64_t* value_strides, tq_dtype in_dtype, int64_t batch,
+                              int32_t heads, int64_t n, int32_t d, const float* krotation,
+                              const float* kboundaries, const float* vrotation,
+                              const float* vboundaries, int32_t vbits, uint8_t* kpairs,
+                              void* knorms, uint8_t* vtiles, void* vnorms, tq_dtype norm_dtype,
+                              int64_t t_cap, int64_t pos, void* stream);
+
+/*
+ * A batch's new keys and values [n_tokens][hkv][64] (bf16 / fp16) quantized and written to
+ * the slots slot_mapping [n_tokens] of decode-layout pools in one launch (kpairs_pool
+ * [num_blocks][hkv][block_size][32], the value tiles and norms of
+ * tq_paged_store_value_tiles): the same bytes as tq_rotate_and_quantize,
+ * tq_pack_decode_layout, tq_paged_store and tq_paged_store_value_tiles.  Slots outside the
+ * pool are skipped.  Pools 16-byte aligned.
+ */
+int tq_paged_write_dl(const void* key, const void* value, tq_dtype in_dtype, int64_t n_tokens,
+                      int32_t hkv, const float* krotation, const float* kboundaries,
+                      const float* vrotation, const float* vboundaries,
+                      const int64_t* slot_mapping, uint8_t* kpairs_pool, float* knorm_pool,
+                      uint8_t* vtile_pool, float* vnorm_pool, int64_t num_blocks,
+                      int32_t block_size, int32_t vbits, void* stream);
+
+/*
  * A decode-layout cache's first T tokens of every (batch row, head) dequantized, followed by
  * n_new tokens copied as they are: keys / values [batch][heads][T + n_new][d] in out_dtype,
  * the tensors the reference's cache hands to a model's attention

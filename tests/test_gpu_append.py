@@ -1,0 +1,91 @@
+"""bf16 / fp16 keys and values quantized straight into decode-layout caches and paged pools
+(csrc/tq_append.hip) against the separate quantize, layout and store ops: the same bytes,
+other tokens' bits untouched."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+
+
+def tables(d, vb):
+    from turboquant_kv.codebook import lloyd_max_codebook, make_rotation_matrix
+    t = lambda x: x.to(DEV)  # noqa: E731
+    return (t(make_rotation_matrix(d, 42)), t(lloyd_max_codebook(4, d)[0]),
+            t(make_rotation_matrix(d, 43)), t(lloyd_max_codebook(vb, d)[0]))
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d,vb", [(64, 2), (64, 3), (64, 4), (128, 2), (128, 3), (128, 4)])
+def test_cache_append(d, vb, dt):
+    """Positions and lengths around the 16-token sub-blocks and 64-token tiles, one token per
+    stream included; contiguous, transposed and unaligned rows; norms in both types."""
+    from turboquant_kv import ops
+    from turboquant_kv._lib import ops as tops
+    Rk, bk, Rv, bv = tables(d, vb)
+    g = torch.Generator(device=DEV).manual_seed(10 * d + vb)
+    cap, B, H = 256, 3, 7
+    for pos, n in ((0, 1), (63, 1), (38, 1), (0, 16), (5, 3), (15, 2), (16, 48), (7, 130), (0, 256), (61, 65)):
+        for form in ("contiguous", "transposed", "odd"):
+            nd = torch.float32 if form == "transposed" else dt
+            new = lambda *s: torch.randint(0, 256, s, generator=g, device=DEV, dtype=torch.uint8)  # noqa: E731
+            kp, vp = new(B, H, cap, d // 2), new(B, H, cap // 64, 8 * vb * d)
+            kn, vn = (torch.randn(B, H, cap, generator=g, device=DEV).to(nd) for _ in range(2))
+            kv = []
+            for _ in range(2):
+                x = torch.randn(B, n, H, d, generator=g, device=DEV).to(dt)
+                x = x.transpose(1, 2)
+                if form == "contiguous":
+                    x = x.contiguous()
+                elif form == "odd":
+                    buf = torch.empty(x.numel() + 1, dtype=dt, device=DEV)[1:].view(B, H, n, d)
+                    x = buf.copy_(x)
+                kv.append(x)
+            want = [t.clone() for t in (kp, kn, vp, vn)]
+            for x, R, b, c, nm, bits, val in ((kv[0], Rk, bk, want[0], want[1], 4, False),
+                                              (kv[1], Rv, bv, want[2], want[3], vb, True)):
+                p, norms = tops().quantize_mse_packed(x.reshape(-1, d), R, b, bits)
+                ops.pack_decode_layout(p.view(B * H, n, -1), c.view(B * H, c.shape[2], -1), d, bits, val, pos)
+                nm[:, :, pos:pos + n] = norms.view(B, H, n).to(nd)
+            tops().cache_append_dl(kv[0], kv[1], kp, kn, vp, vn, pos, Rk, bk, Rv, bv, 4, vb)
+            for got, w, name in zip((kp, kn, vp, vn), want, ("keys", "key norms", "values", "value norms")):
+                assert torch.equal(got, w), (name, pos, n, form)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("block,vb", [(16, 2), (16, 3), (16, 4), (32, 2), (64, 2), (64, 3), (64, 4), (128, 3)])
+def test_paged_write(block, vb, dt):
+    """Slots of prompts (runs from any offset, several sequences in a batch), of decode tokens
+    (scattered), padding and out-of-pool slots; pools keep their other tokens."""
+    from turboquant_kv import ops
+    from turboquant_kv._lib import ops as tops
+    H, nb = 3, 40
+    Rk, bk, Rv, bv = tables(64, vb)
+    g = torch.Generator(device=DEV).manual_seed(block + vb)
+    total = nb * block
+    perm = torch.randperm(total, generator=g, device=DEV)
+    run = lambda a, n: torch.arange(a, a + n, device=DEV)  # noqa: E731
+    pad = torch.tensor([-1, total, total + 5, -7], device=DEV)
+    cases = [perm[:1], perm[:48], run(0, 16), run(0, 37), run(7, 100), run(16, 15), run(33, 16),
+             torch.cat([run(5, 50), run(320, 40), perm[(perm > 400)][:9]]), torch.cat([run(16, 33), pad]),
+             torch.cat([pad, run(48, 64)]), run(0, 32).flip(0),
+             torch.cat([run(0, 8), run(24, 24)]), torch.cat([run(3, 13), pad[:1], run(64, 64)])]
+    for i, slots in enumerate(cases):
+        n = slots.numel()
+        k, v = (torch.randn(n, H, 64, generator=g, device=DEV).to(dt) for _ in range(2))
+        kp = torch.randint(0, 256, (nb, H, block, 32), generator=g, device=DEV, dtype=torch.uint8)
+        shape = (nb, H, block // 64, 512 * vb) if block >= 64 else (nb, H, block // 16, 128 * vb)
+        vt = torch.randint(0, 256, shape, generator=g, device=DEV, dtype=torch.uint8)
+        kn, vn = (torch.randn(nb, H, block, generator=g, device=DEV) for _ in range(2))
+        want = [t.clone() for t in (kp, kn, vt, vn)]
+        kq, knew = tops().quantize_mse_packed(k.reshape(-1, 64), Rk, bk, 4)
+        vq, vnew = tops().quantize_mse_packed(v.reshape(-1, 64), Rv, bv, vb)
+        pairs = torch.empty(n * H, 1, 32, dtype=torch.uint8, device=DEV)
+        ops.pack_decode_layout(kq.view(n * H, 1, -1), pairs, 64, 4, False, 0)
+        ops.paged_store(pairs.view(n, H, -1), knew.float().view(n, H), slots, want[0], want[1])
+        ops.paged_store_value_tiles(vq.view(n, H, -1), vnew.float().view(n, H), slots, want[2], want[3])
+        tops().paged_write_dl(k, v, slots, kp, kn, vt, vn, Rk, bk, Rv, bv)
+        for got, w, name in zip((kp, kn, vt, vn), want, ("keys", "key norms", "values", "value norms")):
+            assert torch.equal(got, w), (name, i)

@@ -1010,6 +1010,47 @@ void paged_store_value_tiles(const at::Tensor& rows, const at::Tensor& norms,
                                       cur_stream(vtile_pool)));
 }
 
+// New keys / values [n, hkv, 64] (bf16 / fp16) quantized and written to their slots of
+// decode-layout pools in one launch (paged_store + paged_store_value_tiles of their codes).
+void paged_write_dl(const at::Tensor& key, const at::Tensor& value, const at::Tensor& slot_mapping,
+                    at::Tensor& kpairs_pool, at::Tensor& knorm_pool, at::Tensor& vtile_pool, at::Tensor& vnorm_pool,
+                    const at::Tensor& krotation, const at::Tensor& kboundaries, const at::Tensor& vrotation,
+                    const at::Tensor& vboundaries) {
+  require_gpu(kpairs_pool, "kpairs_pool");
+  c10::DeviceGuard g(kpairs_pool.device());
+  const auto dev = kpairs_pool.device();
+  TORCH_CHECK(kpairs_pool.dim() == 4 && vtile_pool.dim() == 4 && kpairs_pool.scalar_type() == at::kByte &&
+                  vtile_pool.scalar_type() == at::kByte && kpairs_pool.is_contiguous() && vtile_pool.is_contiguous(),
+              "pools must be contiguous uint8");
+  const int64_t nb = kpairs_pool.size(0), hkv = kpairs_pool.size(1), bs = kpairs_pool.size(2);
+  const int vb = value_tile_bits(vtile_pool.size(3), bs >= 64);
+  TORCH_CHECK(kpairs_pool.size(3) == 32 && vtile_pool.size(0) == nb && vtile_pool.size(1) == hkv &&
+                  vtile_pool.size(2) * (bs >= 64 ? 64 : 16) == bs && vb != 0 && vtile_pool.device() == dev,
+              "decode-layout pool shapes mismatch (head_dim 64)");
+  for (const at::Tensor* t : {&knorm_pool, &vnorm_pool})
+    TORCH_CHECK(t->device() == dev && t->scalar_type() == at::kFloat && t->is_contiguous() &&
+                    t->numel() == nb * hkv * bs,
+                "norm pools must be contiguous float32 [num_blocks, hkv, block_size]");
+  const int64_t n = key.size(0);
+  TORCH_CHECK(key.dim() == 3 && key.size(1) == hkv && key.size(2) == 64 && value.sizes() == key.sizes() &&
+                  value.scalar_type() == key.scalar_type() &&
+                  (key.scalar_type() == at::kBFloat16 || key.scalar_type() == at::kHalf),
+              "key / value must be bfloat16 or float16 [n, hkv, 64]");
+  if (n == 0) return;
+  auto k1 = key.to(dev).contiguous(), v1 = value.to(dev).contiguous();
+  auto sm = slot_mapping.to(dev, at::kLong).contiguous();
+  TORCH_CHECK(sm.numel() == n, "slot_mapping must have one entry per token");
+  auto Rk = f32c(krotation, dev), Rv = f32c(vrotation, dev);
+  auto bk = f32c(kboundaries, dev), bv = f32c(vboundaries, dev);
+  TORCH_CHECK(Rk.numel() == 64 * 64 && Rv.numel() == 64 * 64, "rotations must be [64, 64]");
+  TORCH_CHECK(bk.numel() == 15 && bv.numel() == (1 << vb) - 1, "boundaries length must be 2^bit_width - 1");
+  check_rc(tq_paged_write_dl(k1.data_ptr(), v1.data_ptr(), to_tq(k1.scalar_type()), n, (int32_t)hkv,
+                             Rk.data_ptr<float>(), bk.data_ptr<float>(), Rv.data_ptr<float>(), bv.data_ptr<float>(),
+                             sm.data_ptr<int64_t>(), kpairs_pool.data_ptr<uint8_t>(), knorm_pool.data_ptr<float>(),
+                             vtile_pool.data_ptr<uint8_t>(), vnorm_pool.data_ptr<float>(), nb, (int32_t)bs, vb,
+                             cur_stream(k1)));
+}
+
 std::tuple<at::Tensor, at::Tensor> decode_attention_paged_dl(
     const at::Tensor& q, const at::Tensor& kpairs_pool, const at::Tensor& knorm_pool,
     const at::Tensor& vtile_pool, const at::Tensor& vnorm_pool, const at::Tensor& block_tables,
@@ -1150,6 +1191,31 @@ void cache_append_dl(const at::Tensor& key, const at::Tensor& value, at::Tensor&
   TORCH_CHECK(pos >= 0 && pos + n <= kn.size(2), "tokens past the cache's capacity");
   if (B * H * n == 0) return;
   const auto kdt = key.scalar_type();
+  auto at16 = [](const at::Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; };
+  if (n > 1 && kbits == 4 && vbits >= 2 && vbits <= 4 && (d == 64 || d == 128) &&
+      (kdt == at::kBFloat16 || kdt == at::kHalf) && value.scalar_type() == kdt && kn.is_contiguous() &&
+      vn.is_contiguous() && at16(kp) && at16(vp)) {
+    auto k1 = key.to(dev), v1 = value.to(dev);
+    if (k1.stride(3) != 1) k1 = k1.clone(at::MemoryFormat::Contiguous);
+    if (v1.stride(3) != 1) v1 = v1.clone(at::MemoryFormat::Contiguous);
+    auto Rk = f32c(krotation, dev), Rv = f32c(vrotation, dev);
+    auto bk = f32c(kboundaries, dev), bv = f32c(vboundaries, dev);
+    TORCH_CHECK(Rk.dim() == 2 && Rk.size(0) == d && Rk.size(1) == d && Rv.sizes() == Rk.sizes(),
+                "rotations must be [d, d]");
+    TORCH_CHECK(bk.numel() == 15 && bv.numel() == (1 << vbits) - 1, "boundaries length must be 2^bit_width - 1");
+    TORCH_CHECK(kp.size(3) == d / 2 && vp.size(3) == 8 * vbits * d, "cache width mismatch");
+    const int64_t t_cap = kp.size(2);
+    TORCH_CHECK(vp.size(2) * 64 == t_cap && kn.size(2) == t_cap, "cache capacities differ");
+    const int64_t ks[3] = {k1.stride(0), k1.stride(1), k1.stride(2)}, vs[3] = {v1.stride(0), v1.stride(1), v1.stride(2)};
+    if (at16(Rk) && at16(Rv)) {
+      check_rc(tq_cache_append_tokens_dl(k1.data_ptr(), ks, v1.data_ptr(), vs, to_tq(kdt), B, (int32_t)H, n, (int32_t)d,
+                                         Rk.data_ptr<float>(), bk.data_ptr<float>(), Rv.data_ptr<float>(),
+                                         bv.data_ptr<float>(), (int32_t)vbits, kp.data_ptr<uint8_t>(), kn.data_ptr(),
+                                         vp.data_ptr<uint8_t>(), vn.data_ptr(), to_tq(kn.scalar_type()), t_cap, pos,
+                                         cur_stream(k1)));
+      return;
+    }
+  }
   if (n == 1 && kbits == 4 && vbits >= 2 && vbits <= 4 && (d == 64 || d == 128) &&
       (kdt == at::kBFloat16 || kdt == at::kHalf) && value.scalar_type() == kdt &&
       kn.is_contiguous() && vn.is_contiguous()) {
@@ -1385,6 +1451,9 @@ TORCH_LIBRARY(turboquant, m) {
   m.def("dequantize_cache_dl(Tensor kp, Tensor kn, Tensor vp, Tensor vn, int T, Tensor kcentroids,"
         " Tensor krotation, Tensor vcentroids, Tensor vrotation, ScalarType dtype, Tensor? key_new=None,"
         " Tensor? value_new=None) -> (Tensor, Tensor)");
+  m.def("paged_write_dl(Tensor key, Tensor value, Tensor slot_mapping, Tensor(a!) kpairs_pool,"
+        " Tensor(b!) knorm_pool, Tensor(c!) vtile_pool, Tensor(d!) vnorm_pool, Tensor krotation,"
+        " Tensor kboundaries, Tensor vrotation, Tensor vboundaries) -> ()");
   m.def("paged_store_value_tiles(Tensor rows, Tensor norms, Tensor slot_mapping,"
         " Tensor(a!) vtile_pool, Tensor(b!) vnorm_pool) -> ()");
   m.def("decode_attention_paged_dl(Tensor q, Tensor kpairs_pool, Tensor knorm_pool,"
@@ -1419,6 +1488,7 @@ TORCH_LIBRARY_IMPL(turboquant, CUDA, m) {
   m.impl("paged_gather", &paged_gather);
   m.impl("decode_attention_paged", &decode_attention_paged);
   m.impl("paged_store_value_tiles", &paged_store_value_tiles);
+  m.impl("paged_write_dl", &paged_write_dl);
   m.impl("decode_attention_paged_dl", &decode_attention_paged_dl);
   m.impl("prefill_attention_paged_dl", &prefill_attention_paged_dl);
   m.impl("attention_scores_prod", &attention_scores_prod);

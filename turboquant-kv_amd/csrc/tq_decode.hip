@@ -1600,7 +1600,7 @@ __global__ void dl_pack_kernel(const uint8_t* __restrict__ packed, int64_t n_str
 // One new token per stream quantized and written straight into the decode layout (key
 // pair bytes, the token's bits of its value tile, both norms): a decode step's cache
 // append in one launch instead of a quantize and a layout pass for each of K and V.
-// Arithmetic of quantize_rows_kernel (bf16 / fp16 inputs, rounded in that type), so codes
+// quantize_kernel's arithmetic (bf16 / fp16 inputs, rounded in that type), so codes
 // and norms equal tq_rotate_and_quantize followed by tq_pack_decode_layout bit for bit.
 // One wave per (stream, K or V) row; R_k and R_v, rounded and transposed, in LDS.  A
 // stream's token is the only writer of its bits in this launch: every value-tile byte is
@@ -2324,6 +2324,16 @@ int tq_cache_append_dl(const void* key, const void* value, tq_dtype in_dtype, in
   TQ_REQUIRE(key && value && krotation && kboundaries && vrotation && vboundaries && kpairs &&
                  knorms && vtiles && vnorms,
              "null pointer argument");
+  if (d == 128 && ((reinterpret_cast<uintptr_t>(krotation) | reinterpret_cast<uintptr_t>(vrotation) |
+                    reinterpret_cast<uintptr_t>(kpairs) | reinterpret_cast<uintptr_t>(vtiles)) & 15) == 0) {
+    // 16 streams per wave on the matrix cores: 11.4 us (8 streams, 2-bit values) to 15.4 us
+    // (512, 4-bit) against 15-16.5 us of this file's kernel, whose R_k and R_v (132 KB) leave one
+    // workgroup per CU; at d = 64 it is the faster one (8.3-9.0 us against 8.5-10.8 us)
+    const int64_t strides[3] = {d, 0, 0};
+    return tq_cache_append_tokens_dl(key, strides, value, strides, in_dtype, n_streams, 1, 1, d, krotation,
+                                     kboundaries, vrotation, vboundaries, vbits, kpairs, knorms, vtiles, vnorms,
+                                     norm_dtype, t_cap, pos, stream);
+  }
   AppendArgs a{key, value, (int)in_dtype, n_streams, krotation, kboundaries, vrotation, vboundaries,
                kpairs, knorms, vtiles, vnorms, (int)norm_dtype, t_cap, pos};
   const int64_t want = (2 * n_streams + kApThreads / 64 - 1) / (kApThreads / 64);

@@ -175,6 +175,12 @@ class PagedKVPools:
             self._write_fp(st["k_fp"], key, sm)
             self._write_fp(st["v_fp"], value, sm)
             return
+        if "kp" in st and key.dtype == value.dtype and key.dtype in (torch.bfloat16, torch.float16):
+            # quantized and stored by one launch
+            shape = (n, H, self.head_dim)
+            _ops().paged_write_dl(key.reshape(shape), value.reshape(shape), sm, st["kp"], st["kn"], st["vt"], st["vn"], self.R_k, self.kbnd,
+                                  self.R_v, self.vbnd)
+            return
         kq = self._quantize(key.to(self.device), self.R_k, self.kbnd, self.kcen,
                             getattr(self, "S_k", None), self.config.key_bits)
         vq = self._quantize(value.to(self.device), self.R_v, self.vbnd, self.vcen,
@@ -324,8 +330,12 @@ class PagedKVPools:
         query [num_tokens, Hq, d], key/value [num_tokens, Hkv, d]."""
         layer = md.layer_id
         self.write(layer, key, value, md.slot_mapping)
-        out = output if output is not None else torch.empty_like(query)
         npf = md.num_prefills
+        if npf == 0 and output is None and 0 < query.shape[0] == md.block_tables.shape[0]:
+            # decode tokens only: the kernel's own output is the result
+            return self.decode(layer, query, md.block_tables, md.seq_lens.to(self.device, torch.int32),
+                               scale).to(query)
+        out = output if output is not None else torch.empty_like(query)
         if npf > 0:
             # prefill needs each sequence's token range and context length on the host: the
             # metadata's host copies, else one copy of just the prefill sequences' entries
