@@ -159,6 +159,14 @@ int tq_ip_scan_topk(const void* queries, tq_dtype q_dtype, int64_t nq, int32_t d
                     size_t workspace_bytes, void* stream);
 
 /*
+ * Workspace of tq_ip_scan_topk (prod = pairs = 0), tq_ip_scan_topk_prod (prod = 1) and
+ * tq_ip_scan_topk_prod_pair_rows (prod = pairs = 1) with which they may filter the rows on
+ * the matrix cores; with tq_scan_workspace_bytes they score every row exactly.  Same results.
+ */
+size_t tq_scan_rows_workspace_bytes(int64_t nq, int32_t d, int32_t bit_width, int64_t N, int32_t k,
+                                    int32_t prod, int32_t pairs);
+
+/*
  * The same scan (and tq_attention_scores_packed) over 4-bit rows in the pair layout:
  * row i is d/2 bytes, byte p = code[i][2p] << 4 | code[i][2p+1] -- the bytes of the
  * bit-plane row rearranged, written by tq_pack_decode_layout (values = 0, one stream,

@@ -1,0 +1,115 @@
+"""The filtered row scan (csrc/tq_row_filter.h) against the exact scan: with the workspace of
+tq_scan_workspace_bytes the same entry points score every row exactly, with that of
+tq_scan_rows_workspace_bytes they filter.  Ids and scores agree bit for bit."""
+
+import ctypes
+
+import pytest
+import torch
+
+import capi
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+
+
+def database(N, d, bits, prod, pairs, seed):
+    from turboquant_kv._lib import ops
+    from turboquant_kv.codebook import lloyd_max_codebook, make_qjl_matrix, make_rotation_matrix
+    cb = bits - prod
+    R, S = make_rotation_matrix(d, 42).to(DEV), make_qjl_matrix(d, d, 42).to(DEV)
+    bnd, cen = (t.to(DEV) for t in lloyd_max_codebook(cb, d))
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    x = torch.randn(N, d, generator=g, device=DEV) * torch.exp(torch.randn(N, 1, generator=g, device=DEV) * 0.3)
+    x[100:140] = x[7]  # exact ties
+    x[5] = 0.0
+    if prod:
+        p, sg, rn, nm = ops().quantize_prod_packed(x, R, bnd, cen, S, bits)
+    else:
+        (p, nm), sg, rn = ops().quantize_mse_packed(x, R, bnd, bits), None, None
+    if pairs:
+        p = ops().pack_pair_rows(p, cb, d)
+    return dict(p=p, sg=sg, rn=rn, nm=nm, cen=cen, R=R, S=S, bits=bits, prod=prod, pairs=pairs, d=d, N=N)
+
+
+def scan(db, q, k, filtered):
+    Q, N, d, bits = q.shape[0], db["N"], db["d"], db["bits"]
+    L, c = capi.lib(), capi
+    L.tq_scan_rows_workspace_bytes.restype = ctypes.c_size_t
+    small = L.tq_scan_workspace_bytes(c.i64(Q), c.i32(d), c.i32(bits), c.i64(N), c.i32(k))
+    big = L.tq_scan_rows_workspace_bytes(c.i64(Q), c.i32(d), c.i32(bits), c.i64(N), c.i32(k),
+                                         c.i32(db["prod"]), c.i32(db["pairs"]))
+    ws = torch.empty(big if filtered else small, dtype=torch.uint8, device=DEV)
+    s = torch.empty(Q, k, device=DEV)
+    i = torch.empty(Q, k, dtype=torch.long, device=DEV)
+    dt = {torch.float32: c.TQ_F32, torch.float16: c.TQ_F16, torch.bfloat16: c.TQ_BF16}[q.dtype]
+    tail = (c.i32(bits), c.i32(k), c.p(s), c.p(i), c.p(ws), ctypes.c_size_t(ws.numel()), c.stream())
+    head = (c.p(q), dt, c.i64(Q), c.i32(d), c.p(db["p"]))
+    if db["prod"]:
+        f = L.tq_ip_scan_topk_prod_pair_rows if db["pairs"] else L.tq_ip_scan_topk_prod
+        c.check(f(*head, c.p(db["sg"]), c.p(db["rn"]), c.p(db["nm"]), c.i64(N), c.p(db["cen"]), c.p(db["R"]),
+                  c.p(db["S"]), *tail))
+    else:
+        c.check(L.tq_ip_scan_topk(*head, c.p(db["nm"]), c.i64(N), c.p(db["cen"]), c.p(db["R"]), *tail))
+    return s, i, big > small
+
+
+def same(db, q, k):
+    s0, i0, _ = scan(db, q, k, False)
+    s1, i1, filters = scan(db, q, k, True)
+    assert torch.equal(s0.view(torch.int32), s1.view(torch.int32)) and torch.equal(i0, i1), (db["N"], q.shape, k)
+    return filters
+
+
+@pytest.mark.parametrize("d", [16, 20, 37, 64, 100, 128, 200, 225, 256])
+def test_equals_exact_scan(d):
+    """Dims around the 32-dim steps and byte counts, 2-4 bits, with and without signs, row counts
+    around the 64-row groups and the table's end, 1 to 33 queries, k from 1 to 128, ties."""
+    hit = 0
+    for n, (bits, prod) in enumerate(((2, 0), (3, 0), (4, 0), (3, 1), (4, 1))):
+        for N in (8192, 8193 + 62 * (n % 2), 20_011):
+            db = database(N, d, bits, prod, 0, 10 * d + n)
+            g = torch.Generator(device=DEV).manual_seed(d + n)
+            for Q, k, dt in ((1, 10, torch.float16), (5, 1, torch.float32), (17, 128, torch.bfloat16),
+                             (33, 32, torch.float16)):
+                hit += same(db, torch.randn(Q, d, generator=g, device=DEV).to(dt), k)
+    assert hit >= 40
+
+
+def test_rounds_of_queries():
+    """More queries than one round of lists holds."""
+    db = database(9000, 100, 3, 0, 0, 1)
+    q = torch.randn(600, 100, generator=torch.Generator(device=DEV).manual_seed(2), device=DEV)
+    assert same(db, q, 10)
+
+
+@pytest.mark.parametrize("d,bits", [(64, 3), (64, 4), (128, 3), (128, 4)])
+def test_prod_pair_rows(d, bits):
+    """Prod rows whose codes are pair rows, from where they are filtered."""
+    for N in (120_000, 200_033):
+        db = database(N, d, bits, 1, 1, d + bits)
+        g = torch.Generator(device=DEV).manual_seed(bits)
+        for Q, k in ((64, 10), (40, 100), (130, 33)):
+            assert same(db, torch.randn(Q, d, generator=g, device=DEV).half(), k)
+
+
+@pytest.mark.parametrize("prod", [0, 1])
+def test_special_values(prod):
+    """Zero, infinite and NaN queries, norms and residual norms, and a database of equal rows: the
+    queries the filter cannot bound are answered by the exact scan."""
+    db = database(9000, 200, 4, prod, 0, 3)
+    g = torch.Generator(device=DEV).manual_seed(4)
+    q = torch.randn(18, 200, generator=g, device=DEV)
+    q[1], q[2] = 0.0, q[2] * 1e-30
+    q[3, 5], q[4, 7] = float("inf"), float("nan")
+    q[5] *= 1e30
+    assert same(db, q, 10)
+    db["nm"][::97], db["nm"][50], db["nm"][51] = -1.0, float("inf"), float("nan")
+    if prod:
+        db["rn"][60], db["rn"][61] = float("inf"), float("nan")
+    assert same(db, q, 100)
+    for key in ("p", "sg", "rn", "nm"):
+        if db[key] is not None:
+            db[key][:] = db[key][7].clone()
+    assert same(db, q, 10)

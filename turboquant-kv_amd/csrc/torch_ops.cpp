@@ -336,7 +336,7 @@ std::tuple<at::Tensor, at::Tensor> ip_scan_topk(const at::Tensor& queries, const
   auto os = at::empty({Q, k}, q.options().dtype(at::kFloat));
   auto oi = at::empty({Q, k}, q.options().dtype(at::kLong));
   if (Q == 0) return {os, oi};
-  auto ws = workspace(tq_scan_workspace_bytes(Q, (int32_t)d, (int32_t)bit_width, N, (int32_t)k), dev);
+  auto ws = workspace(tq_scan_rows_workspace_bytes(Q, (int32_t)d, (int32_t)bit_width, N, (int32_t)k, 0, 0), dev);
   check_rc(tq_ip_scan_topk(q.data_ptr(), to_tq(q.scalar_type()), Q, (int32_t)d, p.data_ptr<uint8_t>(),
                            nm.data_ptr<float>(), N, cen.data_ptr<float>(), R.data_ptr<float>(),
                            (int32_t)bit_width, (int32_t)k, os.data_ptr<float>(),
@@ -431,7 +431,7 @@ std::tuple<at::Tensor, at::Tensor> ip_scan_topk_prod_impl(const at::Tensor& quer
   auto os = at::empty({Q, k}, q.options().dtype(at::kFloat));
   auto oi = at::empty({Q, k}, q.options().dtype(at::kLong));
   if (Q == 0) return {os, oi};
-  auto ws = workspace(tq_scan_workspace_bytes(Q, (int32_t)d, (int32_t)bit_width, N, (int32_t)k), dev);
+  auto ws = workspace(tq_scan_rows_workspace_bytes(Q, (int32_t)d, (int32_t)bit_width, N, (int32_t)k, 1, pairs), dev);
   check_rc((pairs ? tq_ip_scan_topk_prod_pair_rows : tq_ip_scan_topk_prod)(
       q.data_ptr(), to_tq(q.scalar_type()), Q, (int32_t)d, r.mp.data_ptr<uint8_t>(),
       r.sg.data_ptr<uint8_t>(), r.rn.data_ptr<float>(), r.nm.data_ptr<float>(), N,

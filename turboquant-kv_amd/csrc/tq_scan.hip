@@ -3273,6 +3273,9 @@ __global__ __launch_bounds__(kMqThreads) void mq_merge_kernel(MqArgs a) {
   for (int e = nvalid_s + tid; e < k; e += kMqThreads) { os[e] = -INFINITY; oi[e] = -1; }
 }
 
+// ------------------------------------------------------------------ filtered row scan
+#include "tq_row_filter.h"
+
 // ------------------------------------------------------------------ softmax stats
 // stats[q] = (max_t s, sum_t exp(s - max)) over the valid tokens of query q's stream.
 __global__ __launch_bounds__(kThreads) void softmax_stats_kernel(const float* __restrict__ scores,
@@ -3792,6 +3795,142 @@ int launch_mq(const void* queries, tq_dtype q_dtype, int64_t nq, int32_t d, cons
   return launch_mq_d<64, 4>(a, L, queries, qbytes, ws, big, st);
 }
 
+// ------------------------------------------------------------------ filtered row scan
+struct RfLayout {
+  int passes, kt, nsgroups, per_bucket, sstride, nbk, nb;
+  size_t qrot, qa, qpar, buckets, tau, flag, cnt, chi, clo, cid, total;
+};
+
+// Queries whose lists (256 x 64 x 12 bytes each) are held at a time: larger calls go in rounds.
+constexpr int64_t kRfRound = 256;
+
+// Offsets past `base`, where the exact scan's lists lie.
+RfLayout rf_layout(int64_t nq, int d, int64_t N, bool prod, size_t base) {
+  RfLayout L{};
+  const int64_t round = std::min(nq, kRfRound);
+  L.passes = (int)((round + kRfQ - 1) / kRfQ);
+  const int bpp = (d + 7) / 8, need = (bpp + 3) / 4;
+  L.kt = need <= 2 ? 2 : need <= 4 ? 4 : need <= 7 ? 7 : 8;
+  const int64_t ngroups = (N + 63) / 64;
+  // a quarter of the rows, 256 to 4,096 groups, in buckets of a group or two: about 4 k rows
+  // (more above a million) reach the k-th largest maximum
+  L.nsgroups = (int)std::min<int64_t>(ngroups, std::min<int64_t>(4096, std::max<int64_t>(256, ngroups / 4)));
+  L.sstride = (int)(ngroups / L.nsgroups);
+  L.per_bucket = (L.nsgroups + kRfMaxBuckets - 1) / kRfMaxBuckets;
+  L.nbk = (L.nsgroups + L.per_bucket - 1) / L.per_bucket;
+  L.nb = filter_blocks(N);
+  const size_t slots = (size_t)L.passes * L.nb * kRfQ;
+  size_t o = align_up(base, 256);
+  auto take = [&](size_t bytes) { const size_t at = o; o = align_up(o + bytes, 256); return at; };
+  L.qrot = take((size_t)round * 256 * 4 * (prod ? 2 : 1));
+  L.qa = take((size_t)L.passes * (prod ? 2 : 1) * L.kt * 1024);
+  L.qpar = take((size_t)L.passes * kRfQ * 16);
+  L.buckets = take((size_t)L.passes * kRfQ * L.nbk * 4);
+  L.tau = take((size_t)L.passes * kRfQ * 4);
+  L.flag = take((size_t)nq * 4);
+  L.cnt = take(slots * 4);
+  L.chi = take(slots * kRfCap * 4);
+  L.clo = take(slots * kRfCap * 4);
+  L.cid = take(slots * kRfCap * 4);
+  L.total = o;
+  return L;
+}
+
+// Where the filtered row scan answers: bit-plane rows of 2-4 bit codes (prod: 2 or 3) and prod
+// pair rows, 8,192 rows or more (shorter calls are a few steps per wave either way).  Times at
+// k = 10 / 100, exact scan -> filtered, in us:
+//   other dims than 64 and 128 (the exact scan's generic loader): always.  200 dims prod, 390,001
+//     rows: 1 query 125 / 171 -> 100 / 115, 16 queries 717 / 698 -> 101 / 117; 10,000 rows, 1
+//     query 115 / 156 -> 73 / 76; 100 dims, 1M rows, 16 queries 516 / 823 -> 79 / 92
+//   bit planes of 64 / 128 dims: from 5 queries, 4 up to a million rows, 2 for k > 32.  128 dims
+//     4 bits, 1M rows: 2 queries 79 / 154 -> 107 / 121, 4 queries 104 / 232 -> 108 / 122, 16
+//     queries 281 / 816 -> 108 / 125; 100,000 rows, 4 queries 86 / 196 -> 65 / 81
+//   prod pair rows (one exact pass per query): from 2 queries, by the exact scan's work.  128 dims,
+//     1M rows: 2 queries 60 / 101 -> 74 / 90, 4 queries 87 / 138 -> 76 / 91, 16 queries 283 /
+//     372 -> 79 / 92; 10M rows, 1 query 157 -> 253, 2 queries 316 -> 267; 10,000 rows, 64
+//     queries 39 / 70 -> 51 / 54
+bool rf_applies(int64_t nq, int d, int64_t N, int k, int bits, bool prod, bool pairs) {
+  if (nq < 1 || nq > INT_MAX || N < 8192 || bits < 2 || bits > (prod ? 3 : 4) || d < 16) return false;
+  const int bpp = (d + 7) / 8;
+  if (pairs) return prod && nq >= 2 && (double)N * nq * d >= (k > kSmallK ? 1.2e8 : 4e8);
+  if (bpp != 8 && bpp != 16) return true;
+  if (k > kSmallK) return nq >= 2;
+  return nq >= 5 || (nq == 4 && N <= 1000000);
+}
+
+template <int BITS, int KT, bool PROD, bool PAIRS>
+int launch_rf_t(const RfArgs& a, const RfLayout& L, hipStream_t st) {
+  const unsigned passes = (unsigned)L.passes;
+  hipLaunchKernelGGL((rf_query_kernel<KT, PROD>), dim3(passes * kRfQ), dim3(PROD ? 512 : 256), 0, st, a);
+  TQ_LAUNCH_CHECK("rf_query_kernel");
+  hipLaunchKernelGGL((rf_sample_kernel<BITS, KT, PROD, PAIRS>), dim3((unsigned)((L.nbk + kRfWaves - 1) / kRfWaves), passes),
+                     dim3(kRfThreads), 0, st, a);
+  TQ_LAUNCH_CHECK("rf_sample_kernel");
+  hipLaunchKernelGGL(rf_tau_kernel, dim3(passes * kRfQ), dim3(kRfThreads), 0, st, a);
+  TQ_LAUNCH_CHECK("rf_tau_kernel");
+  hipLaunchKernelGGL((rf_filter_kernel<BITS, KT, PROD, PAIRS>), dim3((unsigned)L.nb, passes), dim3(kRfThreads), 0, st, a);
+  TQ_LAUNCH_CHECK("rf_filter_kernel");
+  if (a.k > kSmallK)
+    hipLaunchKernelGGL((rf_merge_kernel<BITS, PROD, PAIRS, kRfMergeCapBig>), dim3((unsigned)a.nq), dim3(kRfThreads), 0, st, a);
+  else
+    hipLaunchKernelGGL((rf_merge_kernel<BITS, PROD, PAIRS, kRfMergeCap>), dim3((unsigned)a.nq), dim3(kRfThreads), 0, st, a);
+  TQ_LAUNCH_CHECK("rf_merge_kernel");
+  return TQ_OK;
+}
+
+template <int BITS, bool PROD>
+int launch_rf_bits(const RfArgs& a, const RfLayout& L, bool pairs, hipStream_t st) {
+  if constexpr (PROD) {
+    if (pairs) {
+      if (L.kt == 2) return launch_rf_t<BITS, 2, true, true>(a, L, st);
+      return launch_rf_t<BITS, 4, true, true>(a, L, st);
+    }
+  }
+  switch (L.kt) {
+    case 2: return launch_rf_t<BITS, 2, PROD, false>(a, L, st);
+    case 4: return launch_rf_t<BITS, 4, PROD, false>(a, L, st);
+    case 7: return launch_rf_t<BITS, 7, PROD, false>(a, L, st);
+    default: return launch_rf_t<BITS, 8, PROD, false>(a, L, st);
+  }
+}
+
+// s: the exact scan's arguments (rows, queries, outputs); answers every unflagged query and
+// leaves the flags in *flag.
+int launch_rf(const ScanArgs& s0, int bits, bool pairs, char* ws, const RfLayout& whole, int32_t** flag, hipStream_t st) {
+  *flag = reinterpret_cast<int*>(ws + whole.flag);
+  for (int64_t q0 = 0; q0 < s0.qps; q0 += kRfRound) {
+    ScanArgs s = s0;
+    s.qps = (int)std::min<int64_t>(kRfRound, s0.qps - q0);
+    s.q = static_cast<const char*>(s0.q) + (size_t)q0 * s0.d * dtype_size(s0.q_dt);
+    s.out_s = s0.out_s + (size_t)q0 * s0.k;
+    s.out_i = s0.out_i + (size_t)q0 * s0.k;
+    RfLayout L = whole;
+    L.passes = (s.qps + kRfQ - 1) / kRfQ;
+    RfArgs a{};
+    a.rows = s.packed; a.norms = s.norms; a.signs = s.signs; a.gammas = s.gammas; a.n = s.nrows;
+    a.q = s.q; a.q_dt = s.q_dt; a.nq = s.qps; a.d = s.d; a.bpp = s.bpp; a.bits = bits; a.k = s.k;
+    a.rot = s.rot; a.qjl = s.qjl; a.cen = s.cen; a.qjl_scale = s.qjl_scale;
+    a.qrot = reinterpret_cast<float*>(ws + L.qrot);
+    a.qa = reinterpret_cast<uint32_t*>(ws + L.qa);
+    a.qpar = reinterpret_cast<float4*>(ws + L.qpar);
+    a.buckets = reinterpret_cast<float*>(ws + L.buckets);
+    a.tau = reinterpret_cast<float*>(ws + L.tau);
+    a.flag = *flag + q0;
+    a.cnt = reinterpret_cast<int*>(ws + L.cnt);
+    a.chi = reinterpret_cast<float*>(ws + L.chi);
+    a.clo = reinterpret_cast<float*>(ws + L.clo);
+    a.cid = reinterpret_cast<int*>(ws + L.cid);
+    a.nbk = L.nbk; a.per_bucket = L.per_bucket; a.sstride = L.sstride; a.nsgroups = L.nsgroups; a.nb = L.nb;
+    a.out_s = s.out_s; a.out_i = s.out_i;
+    int rc;
+    if (s.signs) rc = bits == 2 ? launch_rf_bits<2, true>(a, L, pairs, st) : launch_rf_bits<3, true>(a, L, pairs, st);
+    else rc = bits == 2 ? launch_rf_bits<2, false>(a, L, pairs, st) : bits == 3 ? launch_rf_bits<3, false>(a, L, pairs, st)
+                                                                              : launch_rf_bits<4, false>(a, L, pairs, st);
+    if (rc != TQ_OK) return rc;
+  }
+  return TQ_OK;
+}
+
 }  // namespace
 }  // namespace tq
 
@@ -3821,6 +3960,14 @@ size_t tq_scan_pair_rows_workspace_bytes(int64_t nq, int32_t d, int32_t bit_widt
     if (mq > bytes) bytes = mq;
   }
   return bytes;
+}
+
+size_t tq_scan_rows_workspace_bytes(int64_t nq, int32_t d, int32_t bit_width, int64_t N, int32_t k,
+                                    int32_t prod, int32_t pairs) {
+  const size_t bytes = tq_scan_workspace_bytes(nq, d, bit_width, N, k);
+  if (d < 1 || d > 256 || k < 1 || k > kMaxK || !rf_applies(nq, d, N, k, prod ? bit_width - 1 : bit_width, prod, pairs))
+    return bytes;
+  return rf_layout(nq, d, N, prod, bytes).total;
 }
 
 size_t tq_scan_pairs_workspace_bytes(int64_t nq, int32_t d, int64_t N, int32_t k) {
@@ -3888,12 +4035,24 @@ int ip_scan_topk(const void* queries, tq_dtype q_dtype, int64_t nq, int32_t d,
     return launch_filter(queries, q_dtype, nq, d, packed, norms, N, centroids, rotation, k,
                          out_scores, out_ids, static_cast<char*>(workspace) + 256, st);
   TQ_REQUIRE(nq <= 65535 * 4, "too many queries in one call");
-  TQ_REQUIRE(!pairs || (prod ? bit_width - 1 : bit_width) == 4 || nq <= 65535, "too many queries in one call");
+  const int code_bits = prod ? bit_width - 1 : bit_width;
+  TQ_REQUIRE(!pairs || code_bits == 4 || nq <= 65535, "too many queries in one call");
+  // The filtered row scan, when the workspace holds its buffers
+  // (tq_scan_rows_workspace_bytes); the exact scan then answers the queries it flagged.
+  int32_t* flag = nullptr;
+  if (rf_applies(nq, d, N, k, code_bits, prod != nullptr, pairs) && fast_aligned(a)) {
+    const RfLayout L = rf_layout(nq, d, N, prod != nullptr, need);
+    if (workspace_bytes >= L.total && L.nb <= kRfThreads) {
+      const int rc = launch_rf(a, code_bits, pairs, static_cast<char*>(workspace), L, &flag, st);
+      if (rc != TQ_OK) return rc;
+      a.qflag = flag;
+    }
+  }
   int nb = 0;
-  const int rc = launch_scan(a, prod ? bit_width - 1 : bit_width, true, 1, st, pairs, &nb);
+  const int rc = launch_scan(a, code_bits, true, 1, st, pairs, &nb);
   if (rc != TQ_OK) return rc;
   hipLaunchKernelGGL(merge_kernel, dim3((unsigned)nq), dim3(kThreads), 0, st, ps, pi, nb, k,
-                     out_scores, out_ids, (const int32_t*)nullptr);
+                     out_scores, out_ids, (const int32_t*)flag);
   TQ_LAUNCH_CHECK("merge_kernel");
   return TQ_OK;
 }
