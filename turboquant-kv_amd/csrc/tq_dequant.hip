@@ -11,7 +11,10 @@
 // code pairs in LDS, a lane pair's two dims at a time.
 //
 // Why: a vector-ALU contraction of 16-row tiles took 479 us for 262,144 rows of 128 dims,
-// after a pass (140 us) back to bit planes and before a copy (46 us) into the result.
+// after a pass (140 us) back to bit planes and before a copy (46 us) into the result.  Both
+// sides of such a history (4096 tokens, 8 x 8 heads of 128 dims, bf16), one token added to it:
+// 109 us a layer update with the tables' loads waited for one by one and an unroll that
+// spilled 376 bytes a lane, 67 us with neither.
 
 #include "tq_common.h"
 
@@ -57,7 +60,7 @@ struct DqLds {
   alignas(16) uint16_t r16[k16 ? D * (D + 8) + 2 * D : 8];
   float r32[k16 ? 1 : D * (D + 1)];
   static __device__ __forceinline__ int at(int col) { return col * (D + 8) + 32 * (col >> 4); }
-  uint32_t pair[k16 ? 256 : 1][kPairCopies];  // (c[hi nibble], c[lo nibble])
+  alignas(16) uint32_t pair[k16 ? 256 : 1][kPairCopies];  // (c[hi nibble], c[lo nibble])
   float cen[k16 ? 1 : 16][32];
   uint32_t spread[256];                       // kPlanes: a plane byte's bits in eight nibbles
   uint8_t rows[kDqWaves][kDqUnit][D / 2 + 4]; // value tiles as code pairs
@@ -69,65 +72,6 @@ __device__ __forceinline__ void dequant_side(const DqArgs& a, const DqSide& sd, 
   constexpr int KS = D / 32, CT = D / 16;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, c16 = lane & 15;
   const int nlev = 1 << (SRC == kPlanes ? sd.bits : SRC == kKeys ? 4 : SRC);
-
-  // ---- new tokens, copied as they are
-  const int64_t s_new = a.t_out - a.T;
-  if (sd.fresh && s_new > 0) {
-    constexpr int V = 16 / (k16 ? 2 : 4), PR = D / V;  // 16-byte pieces per row
-    constexpr int64_t es = k16 ? 2 : 4;
-    const int64_t total = a.streams * s_new * PR;
-    for (int64_t e = (int64_t)blockIdx.x * kDqThreads + tid; e < total; e += (int64_t)gridDim.x * kDqThreads) {
-      const int pc = (int)(e % PR);
-      const int64_t r = e / PR, s = r / s_new, i = r - s * s_new, b = s / a.heads, h = s - b * a.heads;
-      const char* from = static_cast<const char*>(sd.fresh) + (b * sd.sb + h * sd.sh + i * sd.ss + pc * V) * es;
-      char* to = static_cast<char*>(sd.out) + ((s * a.t_out + a.T + i) * D + pc * V) * es;
-      *reinterpret_cast<v4u*>(to) = *reinterpret_cast<const v4u*>(from);
-    }
-  }
-
-  // ---- tables
-  if constexpr (k16) {
-    for (int e = tid; e < D * D / 8; e += kDqThreads) {  // rows j, j + 1, columns 4 c ..
-      const int j = 2 * (e / (D / 4)), c = 4 * (e % (D / 4));
-      const v4f p = *reinterpret_cast<const v4f*>(sd.rot + j * D + c), q = *reinterpret_cast<const v4f*>(sd.rot + (j + 1) * D + c);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        uint32_t lo, hi;
-        if constexpr (BF) {
-          lo = __float_as_uint(round_bf16(p[i])) >> 16;
-          hi = __float_as_uint(round_bf16(q[i])) >> 16;
-        } else {
-          lo = __builtin_bit_cast(uint16_t, (_Float16)p[i]);
-          hi = __builtin_bit_cast(uint16_t, (_Float16)q[i]);
-        }
-        *reinterpret_cast<uint32_t*>(&t.r16[DqLds<D, OUT>::at(c + i) + j]) = lo | hi << 16;
-      }
-    }
-    for (int e = tid; e < 256 * kPairCopies; e += kDqThreads) {
-      const int idx = e / kPairCopies, hi = idx >> 4, lo = idx & 15;
-      const float ch = hi < nlev ? sd.cen[hi] : 0.f, cl = lo < nlev ? sd.cen[lo] : 0.f;
-      uint32_t h, l;
-      if constexpr (BF) {
-        h = __float_as_uint(round_bf16(ch)) >> 16;
-        l = __float_as_uint(round_bf16(cl)) >> 16;
-      } else {
-        h = __builtin_bit_cast(uint16_t, (_Float16)ch);
-        l = __builtin_bit_cast(uint16_t, (_Float16)cl);
-      }
-      t.pair[idx][e % kPairCopies] = h | l << 16;  // the even dim is the high nibble
-    }
-  } else {
-    for (int e = tid; e < D * D; e += kDqThreads) t.r32[(e % D) * (D + 1) + e / D] = sd.rot[e];
-    for (int e = tid; e < 16 * 32; e += kDqThreads) t.cen[e >> 5][e & 31] = (e >> 5) < nlev ? sd.cen[e >> 5] : 0.f;
-  }
-  if constexpr (SRC == kPlanes) {
-    if (tid < 256) {  // dim i of eight at bit 7 - i; nibbles: the even dim of a byte high
-      uint32_t v = 0;
-      for (int i = 0; i < 8; ++i) v |= ((tid >> (7 - i)) & 1u) << (4 * (i ^ 1));
-      t.spread[tid] = v;
-    }
-  }
-  __syncthreads();
 
   const int64_t per = (a.T + kDqUnit - 1) / kDqUnit, units = a.streams * per;
   const int64_t step = (int64_t)gridDim.x * kDqWaves;
@@ -184,9 +128,61 @@ __device__ __forceinline__ void dequant_side(const DqArgs& a, const DqSide& sd, 
     }
   };
 
+  // ---- tables: everything they are made of requested at once, then the first unit
+  __shared__ float cen_s[16];
+  float cv0 = 0.f;
+  if (tid < nlev) cv0 = sd.cen[tid];
   int64_t unit = (int64_t)blockIdx.x * kDqWaves + wave;
   Raw nx;
-  if (unit < units) load(unit, nx);
+  if constexpr (k16) {
+    constexpr int NP = D * D / 8 / kDqThreads > 0 ? D * D / 8 / kDqThreads : 1;
+    v4f p[NP], q[NP];  // rows j, j + 1, columns 4 c ..
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const int e = i * kDqThreads + tid, j = 2 * (e / (D / 4)), c = 4 * (e % (D / 4));
+      if (e < D * D / 8) {
+        p[i] = *reinterpret_cast<const v4f*>(sd.rot + j * D + c);
+        q[i] = *reinterpret_cast<const v4f*>(sd.rot + (j + 1) * D + c);
+      }
+    }
+    if (unit < units) load(unit, nx);
+    if (tid < 16) cen_s[tid] = cv0;
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const int e = i * kDqThreads + tid, j = 2 * (e / (D / 4)), c = 4 * (e % (D / 4));
+      if (e >= D * D / 8) continue;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        typedef typename std::conditional<BF, __bf16, _Float16>::type h1;
+        typedef h1 h2 __attribute__((ext_vector_type(2)));
+        *reinterpret_cast<uint32_t*>(&t.r16[DqLds<D, OUT>::at(c + k) + j]) =
+            __builtin_bit_cast(uint32_t, (h2){(h1)p[i][k], (h1)q[i][k]});
+      }
+    }
+    __syncthreads();
+    for (int e = tid; e < 256 * kPairCopies / 4; e += kDqThreads) {
+      typedef typename std::conditional<BF, __bf16, _Float16>::type h1;
+      typedef h1 h2 __attribute__((ext_vector_type(2)));
+      const int idx = e / (kPairCopies / 4);  // the even dim is the high nibble
+      const uint32_t v = __builtin_bit_cast(uint32_t, (h2){(h1)cen_s[idx >> 4], (h1)cen_s[idx & 15]});
+      *reinterpret_cast<v4u*>(&t.pair[idx][4 * (e % (kPairCopies / 4))]) = (v4u){v, v, v, v};
+    }
+  } else {
+    if (unit < units) load(unit, nx);
+    if (tid < 16) cen_s[tid] = cv0;
+#pragma unroll 8
+    for (int e = tid; e < D * D; e += kDqThreads) t.r32[(e % D) * (D + 1) + e / D] = sd.rot[e];
+    __syncthreads();
+    for (int e = tid; e < 16 * 32; e += kDqThreads) t.cen[e >> 5][e & 31] = cen_s[e >> 5];
+  }
+  if constexpr (SRC == kPlanes) {
+    if (tid < 256) {  // dim i of eight at bit 7 - i; nibbles: the even dim of a byte high
+      uint32_t v = 0;
+      for (int i = 0; i < 8; ++i) v |= ((tid >> (7 - i)) & 1u) << (4 * (i ^ 1));
+      t.spread[tid] = v;
+    }
+  }
+  __syncthreads();
   for (; unit < units; unit += step) {
     const Raw cur = nx;
     if (unit + step < units) load(unit + step, nx);
@@ -276,6 +272,7 @@ __device__ __forceinline__ void dequant_side(const DqArgs& a, const DqSide& sd, 
       uint16_t* o0 = static_cast<uint16_t*>(sd.out) + (s * a.t_out + tk0) * D + 8 * g;
 #pragma unroll
       for (int p = 0; p < CT / 2; ++p) {
+        __builtin_amdgcn_sched_barrier(0);  // bounds the operand reads in flight (they spilled)
         v4f acc[2][2];  // [token group][column half]
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
@@ -326,6 +323,20 @@ __device__ __forceinline__ void dequant_side(const DqArgs& a, const DqSide& sd, 
         for (int u = 0; u < 2; ++u)
           if ((u ? tk1 : tk0) < a.T) *reinterpret_cast<v4f*>(o0 + u * 16 * D + 16 * ct) = acc[u] * cur.n[u];
       }
+    }
+  }
+  // ---- new tokens, copied as they are
+  const int64_t s_new = a.t_out - a.T;
+  if (sd.fresh && s_new > 0) {
+    constexpr int V = 16 / (k16 ? 2 : 4), PR = D / V;  // 16-byte pieces per row
+    constexpr int64_t es = k16 ? 2 : 4;
+    const int64_t total = a.streams * s_new * PR;
+    for (int64_t e = (int64_t)blockIdx.x * kDqThreads + tid; e < total; e += (int64_t)gridDim.x * kDqThreads) {
+      const int pc = (int)(e % PR);
+      const int64_t r = e / PR, s = r / s_new, i = r - s * s_new, b = s / a.heads, h = s - b * a.heads;
+      const char* from = static_cast<const char*>(sd.fresh) + (b * sd.sb + h * sd.sh + i * sd.ss + pc * V) * es;
+      char* to = static_cast<char*>(sd.out) + ((s * a.t_out + a.T + i) * D + pc * V) * es;
+      *reinterpret_cast<v4u*>(to) = *reinterpret_cast<const v4u*>(from);
     }
   }
 }
