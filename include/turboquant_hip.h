@@ -589,6 +589,16 @@ int tq_prefill_attention_paged_dl(const void* q, tq_dtype q_dtype, int32_t n, in
                                   const float* krotation, const float* vrotation, float scale,
                                   float* out, void* stream);
 
+/* The same with the output [n][hq][64] in out_dtype: TQ_F32 or q_dtype (rounded once). */
+int tq_prefill_attention_paged_dl_out(const void* q, tq_dtype q_dtype, int32_t n, int64_t T, int32_t hq,
+                                  int32_t hkv, int32_t d, const uint8_t* kpairs_pool,
+                                  const float* knorm_pool, const uint8_t* vtile_pool,
+                                  const float* vnorm_pool, int64_t num_blocks, int32_t block_size,
+                                  int32_t vbits, const int32_t* block_table, int32_t max_blocks,
+                                  const float* kcentroids, const float* vcentroids,
+                                  const float* krotation, const float* vrotation, float scale,
+                                  void* out, tq_dtype out_dtype, void* stream);
+
 /*
  * Host-side tables of the reference's standalone C++ core, for TQIX v1 index files
  * (turboquant_core.cpp:559-618), which record only (dim, bit_width, seed): the reader

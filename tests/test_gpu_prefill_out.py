@@ -1,0 +1,42 @@
+"""PagedKVPools.forward's prefill rows: written by the kernel in the result's type, equal to
+the fp32 result rounded once, also where the result is a given tensor, an unaligned one or
+the queries' own memory."""
+import pytest
+import torch
+
+from turboquant_kv.config import TurboQuantConfig
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("how", ["none", "given", "unaligned", "alias"])
+def test_forward_prefill_rows(dtype, how):
+    from turboquant_kv.vllm_plugin import PagedKVPools, TurboQuantAttentionMetadata
+    hkv, hq, d, bs, lens = 2, 6, 64, 16, [97, 33]
+    pools = PagedKVPools(TurboQuantConfig(), 1, 16, bs, hkv, d, DEV, layout="decode")
+    g = torch.Generator(device=DEV).manual_seed(3)
+    n = sum(lens)
+    tables = torch.randperm(16, generator=g, device=DEV).to(torch.int32).view(2, 8)
+    slots = torch.cat([tables[i].long()[torch.arange(t, device=DEV) // bs] * bs + torch.arange(t, device=DEV) % bs
+                       for i, t in enumerate(lens)])
+    q, k, v = (torch.randn(n, h, d, generator=g, device=DEV).to(dtype) for h in (hq, hkv, hkv))
+    md = TurboQuantAttentionMetadata(
+        num_prefills=2, slot_mapping=slots, block_tables=tables,
+        seq_lens=torch.tensor(lens, dtype=torch.int32, device=DEV),
+        query_start_loc=torch.tensor([0, lens[0], n], dtype=torch.int32, device=DEV))
+    out = None
+    if how == "given":
+        out = torch.empty_like(q)
+    elif how == "unaligned":
+        out = torch.empty(q.numel() + 1, dtype=dtype, device=DEV)[1:].view_as(q)
+    pools.write(0, k, v, slots)
+    want = torch.cat([pools.prefill(0, q[a:b], tables[i], b - a, 0.125).to(dtype)
+                      for i, (a, b) in enumerate([(0, lens[0]), (lens[0], n)])])
+    if how == "alias":
+        out = q
+    got = pools.forward(q, k, v, md, 0.125, output=out)
+    if out is not None:
+        assert got.data_ptr() == out.data_ptr()
+    assert got.dtype == dtype and torch.equal(got, want)  # the same sums, rounded once

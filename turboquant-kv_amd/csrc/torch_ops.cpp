@@ -1107,11 +1107,11 @@ std::tuple<at::Tensor, at::Tensor> decode_attention_paged_dl(
   return {out, lse};
 }
 
-at::Tensor prefill_attention_paged_dl(
+at::Tensor prefill_paged_dl(
     const at::Tensor& q, const at::Tensor& kpairs_pool, const at::Tensor& knorm_pool,
     const at::Tensor& vtile_pool, const at::Tensor& vnorm_pool, const at::Tensor& block_table,
     int64_t T, const at::Tensor& kcentroids, const at::Tensor& vcentroids,
-    const at::Tensor& krotation, const at::Tensor& vrotation, double scale) {
+    const at::Tensor& krotation, const at::Tensor& vrotation, double scale, const c10::optional<at::Tensor>& into) {
   require_gpu(q, "q");
   TORCH_CHECK(q.dim() == 3, "q must be [n, Hq, d]");
   TORCH_CHECK(kpairs_pool.dim() == 4 && vtile_pool.dim() == 4,
@@ -1145,14 +1145,38 @@ at::Tensor prefill_attention_paged_dl(
               "decode layout: 4-bit keys (16 centroids) and 2^VB value centroids for the pool's "
               "VB-bit value tiles");
   TORCH_CHECK(Rk.numel() == d * d && Rv.numel() == d * d, "rotations must be [d, d]");
-  auto out = at::empty({n, Hq, d}, qq.options().dtype(at::kFloat));
-  check_rc(tq_prefill_attention_paged_dl(
+  if (into.has_value())
+    TORCH_CHECK(into->device() == dev && into->is_contiguous() && into->sizes() == qq.sizes() &&
+                    into->scalar_type() == qq.scalar_type() &&
+                    reinterpret_cast<uintptr_t>(into->data_ptr()) % 16 == 0,
+                "out must be contiguous, 16-byte aligned, of the query's shape, dtype and device");
+  auto out = into.has_value() ? *into : at::empty({n, Hq, d}, qq.options().dtype(at::kFloat));
+  check_rc(tq_prefill_attention_paged_dl_out(
       qq.data_ptr(), to_tq(qq.scalar_type()), (int32_t)n, T, (int32_t)Hq, (int32_t)Hkv, (int32_t)d,
       kpairs_pool.data_ptr<uint8_t>(), knorm_pool.data_ptr<float>(), vtile_pool.data_ptr<uint8_t>(),
       vnorm_pool.data_ptr<float>(), nb, (int32_t)bs, (int32_t)vb, bt.data_ptr<int32_t>(), (int32_t)bt.numel(),
       kc.data_ptr<float>(), vc.data_ptr<float>(), Rk.data_ptr<float>(), Rv.data_ptr<float>(),
-      (float)scale, out.data_ptr<float>(), cur_stream(qq)));
+      (float)scale, out.data_ptr(), to_tq(out.scalar_type()), cur_stream(qq)));
   return out;
+}
+
+at::Tensor prefill_attention_paged_dl(
+    const at::Tensor& q, const at::Tensor& kpairs_pool, const at::Tensor& knorm_pool,
+    const at::Tensor& vtile_pool, const at::Tensor& vnorm_pool, const at::Tensor& block_table,
+    int64_t T, const at::Tensor& kcentroids, const at::Tensor& vcentroids,
+    const at::Tensor& krotation, const at::Tensor& vrotation, double scale) {
+  return prefill_paged_dl(q, kpairs_pool, knorm_pool, vtile_pool, vnorm_pool, block_table, T, kcentroids, vcentroids,
+                          krotation, vrotation, scale, c10::nullopt);
+}
+
+// The same into `out` [n, Hq, d], of the query's dtype.
+void prefill_attention_paged_dl_out(
+    const at::Tensor& q, const at::Tensor& kpairs_pool, const at::Tensor& knorm_pool,
+    const at::Tensor& vtile_pool, const at::Tensor& vnorm_pool, const at::Tensor& block_table,
+    int64_t T, const at::Tensor& kcentroids, const at::Tensor& vcentroids,
+    const at::Tensor& krotation, const at::Tensor& vrotation, double scale, at::Tensor& out) {
+  prefill_paged_dl(q, kpairs_pool, knorm_pool, vtile_pool, vnorm_pool, block_table, T, kcentroids, vcentroids,
+                   krotation, vrotation, scale, out);
 }
 
 at::Tensor decode_attention_dl(const at::Tensor& q, const at::Tensor& kpairs,
@@ -1464,6 +1488,10 @@ TORCH_LIBRARY(turboquant, m) {
         " Tensor vtile_pool, Tensor vnorm_pool, Tensor block_table, int T,"
         " Tensor kcentroids, Tensor vcentroids, Tensor krotation, Tensor vrotation,"
         " float scale) -> Tensor");
+  m.def("prefill_attention_paged_dl_out(Tensor q, Tensor kpairs_pool, Tensor knorm_pool,"
+        " Tensor vtile_pool, Tensor vnorm_pool, Tensor block_table, int T,"
+        " Tensor kcentroids, Tensor vcentroids, Tensor krotation, Tensor vrotation,"
+        " float scale, Tensor(a!) out) -> ()");
 }
 
 TORCH_LIBRARY_IMPL(turboquant, CUDA, m) {
@@ -1491,6 +1519,7 @@ TORCH_LIBRARY_IMPL(turboquant, CUDA, m) {
   m.impl("paged_write_dl", &paged_write_dl);
   m.impl("decode_attention_paged_dl", &decode_attention_paged_dl);
   m.impl("prefill_attention_paged_dl", &prefill_attention_paged_dl);
+  m.impl("prefill_attention_paged_dl_out", &prefill_attention_paged_dl_out);
   m.impl("attention_scores_prod", &attention_scores_prod);
   m.impl("ip_scan_topk_prod_pair_rows", &ip_scan_topk_prod_pair_rows);
   m.impl("attention_scores_prod_pair_rows", &attention_scores_prod_pair_rows);

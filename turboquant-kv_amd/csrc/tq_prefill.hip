@@ -73,7 +73,8 @@ struct PfArgs {
   const float* krot;  // [64][64]
   const float* vrot;
   float qscale;  // softmax scale * log2(e)
-  float* out;    // [n][hq][64]
+  void* out;     // [n][hq][64], out_dt
+  int out_dt;    // TQ_F32, or q_dt
 };
 
 __device__ __forceinline__ pf_v8h pf_h8(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
@@ -557,7 +558,6 @@ __global__ __launch_bounds__(kPfThreads, 2) void dl_prefill_kernel(PfArgs a) {
     lt += __shfl_xor(lt, 16, 64);
     lt += __shfl_xor(lt, 32, 64);
     const float inv = lt > 0.f ? 1.f / (lt * vsc) * vs.inv() : 0.f;
-    float* dst = a.out + qoff[j];
 #pragma unroll
     for (int ob = 0; ob < 4; ++ob) {
       pf_v4f acc = (pf_v4f){0.f, 0.f, 0.f, 0.f};
@@ -566,7 +566,17 @@ __global__ __launch_bounds__(kPfThreads, 2) void dl_prefill_kernel(PfArgs a) {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
           acc = __builtin_amdgcn_mfma_f32_16x16x4f32(rv[ob][4 * nb + r], o[j][nb][r] * inv, acc, 0, 0, 0);
-      if (row[j] < nG) *reinterpret_cast<pf_v4f*>(dst + 16 * ob + 4 * g) = acc;
+      if (row[j] >= nG) continue;
+      const int64_t at = qoff[j] + 16 * ob + 4 * g;
+      if (a.out_dt == TQ_F32) {
+        *reinterpret_cast<pf_v4f*>(static_cast<float*>(a.out) + at) = acc;
+      } else if (a.out_dt == TQ_BF16) {
+        typedef __bf16 b4_t __attribute__((ext_vector_type(4)));
+        *reinterpret_cast<b4_t*>(static_cast<uint16_t*>(a.out) + at) = __builtin_convertvector(acc, b4_t);
+      } else {
+        typedef _Float16 h4_t __attribute__((ext_vector_type(4)));
+        *reinterpret_cast<h4_t*>(static_cast<uint16_t*>(a.out) + at) = __builtin_convertvector(acc, h4_t);
+      }
     }
   }
 }
@@ -593,6 +603,20 @@ int tq_prefill_attention_paged_dl(const void* q, tq_dtype q_dtype, int32_t n, in
                                   const float* kcentroids, const float* vcentroids,
                                   const float* krotation, const float* vrotation, float scale,
                                   float* out, void* stream) {
+  return tq_prefill_attention_paged_dl_out(q, q_dtype, n, T, hq, hkv, d, kpairs_pool, knorm_pool, vtile_pool,
+                                           vnorm_pool, num_blocks, block_size, vbits, block_table, max_blocks,
+                                           kcentroids, vcentroids, krotation, vrotation, scale, out, TQ_F32, stream);
+}
+
+int tq_prefill_attention_paged_dl_out(const void* q, tq_dtype q_dtype, int32_t n, int64_t T, int32_t hq,
+                                      int32_t hkv, int32_t d, const uint8_t* kpairs_pool,
+                                      const float* knorm_pool, const uint8_t* vtile_pool,
+                                      const float* vnorm_pool, int64_t num_blocks, int32_t block_size,
+                                      int32_t vbits, const int32_t* block_table, int32_t max_blocks,
+                                      const float* kcentroids, const float* vcentroids,
+                                      const float* krotation, const float* vrotation, float scale,
+                                      void* out, tq_dtype out_dtype, void* stream) {
+  TQ_REQUIRE(out_dtype == TQ_F32 || out_dtype == q_dtype, "the output is float32 or the query's type");
   TQ_REQUIRE(valid_dtype(q_dtype), "unknown dtype");
   TQ_REQUIRE(d == 64, "decode layout covers head_dim 64, got %d", d);
   TQ_REQUIRE(vbits >= 2 && vbits <= 4, "value tiles hold 2-4 bit codes, got %d", vbits);
@@ -633,6 +657,7 @@ int tq_prefill_attention_paged_dl(const void* q, tq_dtype q_dtype, int32_t n, in
   a.kcen = kcentroids; a.vcen = vcentroids; a.krot = krotation; a.vrot = vrotation;
   a.qscale = scale * 1.4426950408889634f;
   a.out = out;
+  a.out_dt = (int)out_dtype;
   const dim3 gr((unsigned)grid);
   hipStream_t st = as_stream(stream);
   if (bsl >= 6) {
