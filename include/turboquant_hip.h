@@ -459,6 +459,19 @@ int tq_decode_attention_dl_window(const void* q, tq_dtype q_dtype, int32_t B, in
                                   const float* vrotation, int32_t kbits, int32_t vbits,
                                   float scale, void* out, float* lse, void* workspace,
                                   size_t workspace_bytes, void* stream);
+/*
+ * The same over the first len tokens (0 <= len <= t_cap) of every sequence: no length tensor,
+ * and the splits are planned for len; workspace: tq_decode_dl_workspace_bytes of len rounded
+ * up to a multiple of 64 (at least 64).
+ */
+int tq_decode_attention_dl_len(const void* q, tq_dtype q_dtype, int32_t B, int32_t hq, int32_t hkv,
+                               int32_t d, const uint8_t* kpairs, const void* knorms,
+                               const uint8_t* vblocks, const void* vnorms, tq_dtype norm_dtype,
+                               int64_t t_cap, int64_t len, const float* kcentroids,
+                               const float* vcentroids, const float* krotation,
+                               const float* vrotation, int32_t kbits, int32_t vbits, float scale,
+                               void* out, float* lse, void* workspace, size_t workspace_bytes,
+                               void* stream);
 
 /*
  * The exact current token merged into a decode output (o, lse from

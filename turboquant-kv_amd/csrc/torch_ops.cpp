@@ -903,9 +903,10 @@ at::Tensor unpack_decode_layout(const at::Tensor& cache, int64_t dim, int64_t bi
   return out;
 }
 
-std::tuple<at::Tensor, at::Tensor> decode_attention_dl_lse(
+// seq_lens: the sequences' lengths; null: `length` tokens in each.
+std::tuple<at::Tensor, at::Tensor> decode_dl(
     const at::Tensor& q, const at::Tensor& kpairs, const at::Tensor& knorms,
-    const at::Tensor& vblocks, const at::Tensor& vnorms, const at::Tensor& seq_lens,
+    const at::Tensor& vblocks, const at::Tensor& vnorms, const at::Tensor* seq_lens, int64_t length,
     const at::Tensor& kcentroids, const at::Tensor& vcentroids, const at::Tensor& krotation,
     const at::Tensor& vrotation, double scale, const c10::optional<at::Tensor>& seq_starts) {
   require_gpu(q, "q");
@@ -936,8 +937,13 @@ std::tuple<at::Tensor, at::Tensor> decode_attention_dl_lse(
                   vnorms.scalar_type() == ndt && knorms.numel() == B * Hkv * Tc &&
                   vnorms.numel() == B * Hkv * Tc,
               "norms must be [B, Hkv, T], both float32, bfloat16 or float16");
-  auto sl = seq_lens.to(dev, at::kInt).contiguous();
-  TORCH_CHECK(sl.numel() == B, "seq_lens must have B entries");
+  at::Tensor sl;
+  if (seq_lens) {
+    sl = seq_lens->to(dev, at::kInt).contiguous();
+    TORCH_CHECK(sl.numel() == B, "seq_lens must have B entries");
+  } else {
+    TORCH_CHECK(length >= 0 && length <= Tc, "length ", length, " outside the capacity ", Tc);
+  }
   at::Tensor ss;
   if (seq_starts.has_value() && seq_starts->defined()) {
     ss = seq_starts->to(dev, at::kInt).contiguous();
@@ -952,6 +958,17 @@ std::tuple<at::Tensor, at::Tensor> decode_attention_dl_lse(
   auto out = at::empty({B, Hq, d}, qq.options());
   auto lse = at::empty({B, Hq}, qq.options().dtype(at::kFloat));
   if (B == 0) return {out, lse};
+  if (!seq_lens) {
+    auto ws = workspace(tq_decode_dl_workspace_bytes((int32_t)B, (int32_t)Hq, (int32_t)Hkv,
+                                                     std::max<int64_t>(64, (length + 63) / 64 * 64)), dev);
+    check_rc(tq_decode_attention_dl_len(
+        qq.data_ptr(), to_tq(qq.scalar_type()), (int32_t)B, (int32_t)Hq, (int32_t)Hkv, (int32_t)d,
+        kpairs.data_ptr<uint8_t>(), knorms.data_ptr(), vblocks.data_ptr<uint8_t>(),
+        vnorms.data_ptr(), to_tq(ndt), Tc, length, kc.data_ptr<float>(), vc.data_ptr<float>(),
+        Rk.data_ptr<float>(), Rv.data_ptr<float>(), 4, (int32_t)vbits, (float)scale,
+        out.data_ptr(), lse.data_ptr<float>(), ws.data_ptr(), ws.numel(), cur_stream(qq)));
+    return {out, lse};
+  }
   auto ws = workspace(tq_decode_dl_workspace_bytes((int32_t)B, (int32_t)Hq, (int32_t)Hkv, Tc), dev);
   check_rc(tq_decode_attention_dl_window(
       qq.data_ptr(), to_tq(qq.scalar_type()), (int32_t)B, (int32_t)Hq, (int32_t)Hkv, (int32_t)d,
@@ -962,6 +979,15 @@ std::tuple<at::Tensor, at::Tensor> decode_attention_dl_lse(
       (float)scale, out.data_ptr(), lse.data_ptr<float>(), ws.data_ptr(), ws.numel(),
       cur_stream(qq)));
   return {out, lse};
+}
+
+std::tuple<at::Tensor, at::Tensor> decode_attention_dl_lse(
+    const at::Tensor& q, const at::Tensor& kpairs, const at::Tensor& knorms,
+    const at::Tensor& vblocks, const at::Tensor& vnorms, const at::Tensor& seq_lens,
+    const at::Tensor& kcentroids, const at::Tensor& vcentroids, const at::Tensor& krotation,
+    const at::Tensor& vrotation, double scale, const c10::optional<at::Tensor>& seq_starts) {
+  return decode_dl(q, kpairs, knorms, vblocks, vnorms, &seq_lens, -1, kcentroids, vcentroids, krotation,
+                   vrotation, scale, seq_starts);
 }
 
 // Value widths of decode-layout value pools: tile_bytes = 64-token tiles of 512 * VB bytes
@@ -1177,6 +1203,17 @@ void prefill_attention_paged_dl_out(
     const at::Tensor& krotation, const at::Tensor& vrotation, double scale, at::Tensor& out) {
   prefill_paged_dl(q, kpairs_pool, knorm_pool, vtile_pool, vnorm_pool, block_table, T, kcentroids, vcentroids,
                    krotation, vrotation, scale, out);
+}
+
+// Every sequence's first `length` tokens.
+at::Tensor decode_attention_dl_len(const at::Tensor& q, const at::Tensor& kpairs,
+                                   const at::Tensor& knorms, const at::Tensor& vblocks,
+                                   const at::Tensor& vnorms, int64_t length,
+                                   const at::Tensor& kcentroids, const at::Tensor& vcentroids,
+                                   const at::Tensor& krotation, const at::Tensor& vrotation,
+                                   double scale) {
+  return std::get<0>(decode_dl(q, kpairs, knorms, vblocks, vnorms, nullptr, length, kcentroids, vcentroids,
+                               krotation, vrotation, scale, c10::nullopt));
 }
 
 at::Tensor decode_attention_dl(const at::Tensor& q, const at::Tensor& kpairs,
@@ -1459,6 +1496,9 @@ TORCH_LIBRARY(turboquant, m) {
   m.def("decode_attention_dl(Tensor q, Tensor kpairs, Tensor knorms, Tensor vblocks,"
         " Tensor vnorms, Tensor seq_lens, Tensor kcentroids, Tensor vcentroids,"
         " Tensor krotation, Tensor vrotation, float scale) -> Tensor");
+  m.def("decode_attention_dl_len(Tensor q, Tensor kpairs, Tensor knorms, Tensor vblocks,"
+        " Tensor vnorms, int length, Tensor kcentroids, Tensor vcentroids,"
+        " Tensor krotation, Tensor vrotation, float scale) -> Tensor");
   m.def("decode_attention_dl_lse(Tensor q, Tensor kpairs, Tensor knorms, Tensor vblocks,"
         " Tensor vnorms, Tensor seq_lens, Tensor kcentroids, Tensor vcentroids,"
         " Tensor krotation, Tensor vrotation, float scale, Tensor? seq_starts=None)"
@@ -1528,6 +1568,7 @@ TORCH_LIBRARY_IMPL(turboquant, CUDA, m) {
   m.impl("pack_decode_layout", &pack_decode_layout);
   m.impl("unpack_decode_layout", &unpack_decode_layout);
   m.impl("decode_attention_dl", &decode_attention_dl);
+  m.impl("decode_attention_dl_len", &decode_attention_dl_len);
   m.impl("decode_attention_dl_lse", &decode_attention_dl_lse);
   m.impl("decode_merge_token", &decode_merge_token);
   m.impl("decode_attention_dl_merged", &decode_attention_dl_merged);

@@ -465,7 +465,8 @@ __global__ __launch_bounds__(D) void fused_combine_kernel(const float* __restric
   float rcol[D];
 #pragma unroll
   for (int k = 0; k < D; ++k) rcol[k] = vrot[k * D + j];
-  const int64_t T = min((int64_t)max(seq_lens[b], 0), t_max);
+  // (no seq_lens: every sequence has t_max tokens)
+  const int64_t T = seq_lens ? min((int64_t)max(seq_lens[b], 0), t_max) : t_max;
   const int ns = (int)((T + split_tokens - 1) / split_tokens);
   float M = -INFINITY;
   for (int s = 0; s < ns; ++s) M = fmaxf(M, stats[row * nsplit + s].x);
@@ -526,7 +527,8 @@ struct DlArgs {
   const uint8_t* vblocks;  // [B*hkv][t_cap/4][64]
   const float* vnorms;
   int64_t t_cap;
-  const int32_t* seq_lens;
+  const int32_t* seq_lens;  // null: len tokens in every sequence
+  int32_t len;
   // optional [B]: tokens before seq_starts[b] are masked (left-padded batches); the
   // tiles holding them are still read
   const int32_t* seq_starts;
@@ -693,7 +695,7 @@ __global__ __launch_bounds__(kDlThreads, 1) void dl_decode_kernel(DlArgs a) {
   // The sequence length is requested first, and nothing below is addressed through it
   // until the prologue's loads (query, R_k, the first tiles) are all in flight: their
   // latency and its own then overlap instead of following one another.
-  const int32_t slen = live ? a.seq_lens[b] : 0;
+  const int32_t slen = !live ? 0 : a.seq_lens ? a.seq_lens[b] : a.len;
   const int32_t sstart = a.seq_starts ? a.seq_starts[b] : 0;
   const int64_t t_begin = (int64_t)split * a.split_tokens;
   const int64_t qh0 = (int64_t)b * a.hq + (int64_t)g * a.Gfull + a.hofs;
@@ -2118,11 +2120,11 @@ int run_dl(DlArgs a, tq_dtype q_dtype, int B, int hq, int hkv, int vbits, int pg
   }
   if (d == 128)
     hipLaunchKernelGGL(fused_combine_kernel<128>, dim3((unsigned)rows), dim3(128), 0, st, part, stats,
-                       p.nsplit, p.split_tokens, a.seq_lens, a.t_cap, hq, a.vrot, (int)q_dtype, out,
+                       p.nsplit, p.split_tokens, a.seq_lens, a.seq_lens ? a.t_cap : (int64_t)a.len, hq, a.vrot, (int)q_dtype, out,
                        lse);
   else
     hipLaunchKernelGGL(fused_combine_kernel<kDim>, dim3((unsigned)rows), dim3(kDim), 0, st, part, stats,
-                       p.nsplit, p.split_tokens, a.seq_lens, a.t_cap, hq, a.vrot, (int)q_dtype, out,
+                       p.nsplit, p.split_tokens, a.seq_lens, a.seq_lens ? a.t_cap : (int64_t)a.len, hq, a.vrot, (int)q_dtype, out,
                        lse);
   TQ_LAUNCH_CHECK("fused_combine_kernel");
   return TQ_OK;
@@ -2132,6 +2134,56 @@ int run_dl(DlArgs a, tq_dtype q_dtype, int B, int hq, int hkv, int vbits, int pg
 }  // namespace tq
 
 using namespace tq;
+
+namespace {
+
+int decode_dl(const void* q, tq_dtype q_dtype, int32_t B, int32_t hq,
+              int32_t hkv, int32_t d, const uint8_t* kpairs,
+              const void* knorms, const uint8_t* vblocks,
+              const void* vnorms, tq_dtype norm_dtype, int64_t t_cap,
+              const int32_t* seq_lens, int64_t len,
+              const int32_t* seq_starts, const float* kcentroids,
+              const float* vcentroids, const float* krotation,
+              const float* vrotation, int32_t kbits, int32_t vbits,
+              float scale, void* out, float* lse, void* workspace,
+              size_t workspace_bytes, void* stream) {
+  TQ_REQUIRE(valid_dtype(q_dtype) && valid_dtype(norm_dtype), "unknown dtype");
+  if ((d != 64 && d != 128) || kbits != 4 || vbits < 2 || vbits > 4)
+    return fail(TQ_EUNSUPPORTED, "decode layout covers head_dim 64 and 128 with 4-bit keys and "
+                                 "2-4 bit values, got d=%d kbits=%d vbits=%d", d, kbits, vbits);
+  TQ_REQUIRE(B >= 0 && hkv >= 1 && hq >= hkv && hq % hkv == 0,
+             "num_heads (%d) must be a multiple of num_kv_heads (%d)", hq, hkv);
+  TQ_REQUIRE(t_cap >= 0 && t_cap % 64 == 0, "capacity must be a multiple of 64, got %lld",
+             (long long)t_cap);
+  TQ_REQUIRE(t_cap * (d / 2) < (int64_t)INT_MAX, "capacity too large for 32-bit offsets");
+  if (B == 0) return TQ_OK;
+  TQ_REQUIRE(seq_lens || (len >= 0 && len <= t_cap), "length %lld outside the capacity %lld", (long long)len,
+             (long long)t_cap);
+  TQ_REQUIRE(q && out && kcentroids && vcentroids && krotation && vrotation,
+             "null pointer argument");
+  TQ_REQUIRE(t_cap == 0 || (kpairs && knorms && vblocks && vnorms), "null pointer argument");
+  TQ_REQUIRE(((reinterpret_cast<uintptr_t>(krotation) | reinterpret_cast<uintptr_t>(vrotation)) & 15u) == 0,
+             "rotations must be 16-byte aligned");
+  TQ_REQUIRE(t_cap == 0 || ((reinterpret_cast<uintptr_t>(kpairs) | reinterpret_cast<uintptr_t>(vblocks) |
+                             reinterpret_cast<uintptr_t>(knorms) | reinterpret_cast<uintptr_t>(vnorms)) &
+                            15u) == 0,
+             "decode-layout K/V and norms must be 16-byte aligned");
+  // a length known here plans the splits for its own tokens, not for the capacity's
+  const int64_t t_plan = seq_lens ? t_cap : std::max<int64_t>(64, (len + 63) & ~(int64_t)63);
+  const size_t need = tq_decode_dl_workspace_bytes(B, hq, hkv, t_plan);
+  TQ_REQUIRE(workspace && workspace_bytes >= need, "workspace too small: need %zu bytes", need);
+  const SplitPlan p = t_cap > 0 ? plan_dl_splits(B, hkv, t_plan) : SplitPlan{kDlMinSplit, 1};
+  DlArgs a{};
+  a.q = q; a.kpairs = kpairs; a.knorms = static_cast<const float*>(knorms); a.vblocks = vblocks;
+  a.vnorms = static_cast<const float*>(vnorms); a.t_cap = t_cap; a.seq_lens = seq_lens;
+  a.len = seq_lens ? 0 : (int32_t)len;
+  a.seq_starts = seq_starts; a.kcen = kcentroids; a.vcen = vcentroids; a.krot = krotation;
+  a.vrot = vrotation; a.qscale = scale * 1.4426950408889634f;
+  return run_dl(a, q_dtype, B, hq, hkv, vbits, 0, p, workspace, out, lse, as_stream(stream),
+                (int)norm_dtype, d);
+}
+
+}  // namespace
 
 extern "C" {
 
@@ -2153,35 +2205,22 @@ int tq_decode_attention_dl_window(const void* q, tq_dtype q_dtype, int32_t B, in
                                   const float* vrotation, int32_t kbits, int32_t vbits,
                                   float scale, void* out, float* lse, void* workspace,
                                   size_t workspace_bytes, void* stream) {
-  TQ_REQUIRE(valid_dtype(q_dtype) && valid_dtype(norm_dtype), "unknown dtype");
-  if ((d != 64 && d != 128) || kbits != 4 || vbits < 2 || vbits > 4)
-    return fail(TQ_EUNSUPPORTED, "decode layout covers head_dim 64 and 128 with 4-bit keys and "
-                                 "2-4 bit values, got d=%d kbits=%d vbits=%d", d, kbits, vbits);
-  TQ_REQUIRE(B >= 0 && hkv >= 1 && hq >= hkv && hq % hkv == 0,
-             "num_heads (%d) must be a multiple of num_kv_heads (%d)", hq, hkv);
-  TQ_REQUIRE(t_cap >= 0 && t_cap % 64 == 0, "capacity must be a multiple of 64, got %lld",
-             (long long)t_cap);
-  TQ_REQUIRE(t_cap * (d / 2) < (int64_t)INT_MAX, "capacity too large for 32-bit offsets");
-  if (B == 0) return TQ_OK;
-  TQ_REQUIRE(q && out && seq_lens && kcentroids && vcentroids && krotation && vrotation,
-             "null pointer argument");
-  TQ_REQUIRE(t_cap == 0 || (kpairs && knorms && vblocks && vnorms), "null pointer argument");
-  TQ_REQUIRE(((reinterpret_cast<uintptr_t>(krotation) | reinterpret_cast<uintptr_t>(vrotation)) & 15u) == 0,
-             "rotations must be 16-byte aligned");
-  TQ_REQUIRE(t_cap == 0 || ((reinterpret_cast<uintptr_t>(kpairs) | reinterpret_cast<uintptr_t>(vblocks) |
-                             reinterpret_cast<uintptr_t>(knorms) | reinterpret_cast<uintptr_t>(vnorms)) &
-                            15u) == 0,
-             "decode-layout K/V and norms must be 16-byte aligned");
-  const size_t need = tq_decode_dl_workspace_bytes(B, hq, hkv, t_cap);
-  TQ_REQUIRE(workspace && workspace_bytes >= need, "workspace too small: need %zu bytes", need);
-  const SplitPlan p = t_cap > 0 ? plan_dl_splits(B, hkv, t_cap) : SplitPlan{kDlMinSplit, 1};
-  DlArgs a{};
-  a.q = q; a.kpairs = kpairs; a.knorms = static_cast<const float*>(knorms); a.vblocks = vblocks;
-  a.vnorms = static_cast<const float*>(vnorms); a.t_cap = t_cap; a.seq_lens = seq_lens;
-  a.seq_starts = seq_starts; a.kcen = kcentroids; a.vcen = vcentroids; a.krot = krotation;
-  a.vrot = vrotation; a.qscale = scale * 1.4426950408889634f;
-  return run_dl(a, q_dtype, B, hq, hkv, vbits, 0, p, workspace, out, lse, as_stream(stream),
-                (int)norm_dtype, d);
+  TQ_REQUIRE(seq_lens || B <= 0, "null pointer argument");
+  return decode_dl(q, q_dtype, B, hq, hkv, d, kpairs, knorms, vblocks, vnorms, norm_dtype, t_cap, seq_lens, -1,
+                   seq_starts, kcentroids, vcentroids, krotation, vrotation, kbits, vbits, scale, out, lse,
+                   workspace, workspace_bytes, stream);
+}
+
+int tq_decode_attention_dl_len(const void* q, tq_dtype q_dtype, int32_t B, int32_t hq, int32_t hkv,
+                               int32_t d, const uint8_t* kpairs, const void* knorms,
+                               const uint8_t* vblocks, const void* vnorms, tq_dtype norm_dtype,
+                               int64_t t_cap, int64_t len, const float* kcentroids,
+                               const float* vcentroids, const float* krotation, const float* vrotation,
+                               int32_t kbits, int32_t vbits, float scale, void* out, float* lse,
+                               void* workspace, size_t workspace_bytes, void* stream) {
+  return decode_dl(q, q_dtype, B, hq, hkv, d, kpairs, knorms, vblocks, vnorms, norm_dtype, t_cap, nullptr, len,
+                   nullptr, kcentroids, vcentroids, krotation, vrotation, kbits, vbits, scale, out, lse,
+                   workspace, workspace_bytes, stream);
 }
 
 int tq_decode_attention_dl(const void* q, tq_dtype q_dtype, int32_t B, int32_t hq, int32_t hkv,

@@ -335,10 +335,16 @@ class QuantizedKVCache:
             raise ValueError(f"query batch {B} != cache batch_size {self.batch_size}")
         if scale is None:
             scale = 1.0 / math.sqrt(self.head_dim)
+        dl = self._dl and q.shape[1] % self.num_heads == 0
         if seq_lens is None:
-            seq_lens = torch.full((B,), int(self.seq_lens[layer_id].item()), dtype=torch.int32,
-                                  device=self.device)
-        if self._dl and q.shape[1] % self.num_heads == 0:
+            T = int(self.seq_lens[layer_id].item())
+            if dl:  # the length as an argument: no tensor of lengths to fill (4 us a call)
+                return ops.decode_attention_dl_len(
+                    q, self._kstore[layer_id], self._key_norms[layer_id], self._vstore[layer_id],
+                    self._val_norms[layer_id], T, self._kcen, self._vcen, self._key_rotation,
+                    self._val_rotation, scale)
+            seq_lens = torch.full((B,), T, dtype=torch.int32, device=self.device)
+        if dl:
             return ops.decode_attention_dl(
                 q, self._kstore[layer_id], self._key_norms[layer_id], self._vstore[layer_id],
                 self._val_norms[layer_id], seq_lens, self._kcen, self._vcen, self._key_rotation,

@@ -178,6 +178,14 @@ def decode_attention_dl(q, kpairs, knorms, vblocks, vnorms, seq_lens, kcentroids
                                       vcentroids, krotation, vrotation, float(scale))
 
 
+def decode_attention_dl_len(q, kpairs, knorms, vblocks, vnorms, length, kcentroids, vcentroids,
+                            krotation, vrotation, scale):
+    """decode_attention_dl over the first `length` tokens of every sequence."""
+    _require_device(q, "q")
+    return _ops().decode_attention_dl_len(q, kpairs, knorms, vblocks, vnorms, int(length), kcentroids,
+                                          vcentroids, krotation, vrotation, float(scale))
+
+
 def paged_store(rows, norms, slot_mapping, pool, norm_pool):
     """Scatter rows [n, hkv, P] (+ norms [n, hkv]) to the flat slots slot_mapping [n] of a
     block pool [num_blocks, hkv, block_size, P] (+ [num_blocks, hkv, block_size]); slots
