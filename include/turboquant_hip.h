@@ -485,6 +485,20 @@ int tq_decode_attention_dl_len(const void* q, tq_dtype q_dtype, int32_t B, int32
 int tq_decode_merge_token(const void* o, const float* lse, const void* q, tq_dtype q_dtype,
                           const void* k_new, const void* v_new, tq_dtype kv_dtype, int32_t B,
                           int32_t hq, int32_t hkv, int32_t d, float scale, void* out, void* stream);
+/*
+ * tq_decode_attention_dl_window followed by tq_decode_merge_token, the merge done as the
+ * output is stored (no launch of its own); the same result.  out must not be q, k_new or v_new.
+ */
+int tq_decode_attention_dl_merged(const void* q, tq_dtype q_dtype, int32_t B, int32_t hq,
+                                  int32_t hkv, int32_t d, const uint8_t* kpairs,
+                                  const void* knorms, const uint8_t* vblocks,
+                                  const void* vnorms, tq_dtype norm_dtype, int64_t t_cap,
+                                  const int32_t* seq_lens, const int32_t* seq_starts,
+                                  const float* kcentroids, const float* vcentroids,
+                                  const float* krotation, const float* vrotation, int32_t kbits,
+                                  int32_t vbits, float scale, const void* k_new, const void* v_new,
+                                  tq_dtype kv_dtype, void* out, void* workspace,
+                                  size_t workspace_bytes, void* stream);
 
 /*
  * Paged KV storage (vLLM block tables).  The reference's vLLM backend keeps one

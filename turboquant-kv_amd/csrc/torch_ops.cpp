@@ -903,12 +903,15 @@ at::Tensor unpack_decode_layout(const at::Tensor& cache, int64_t dim, int64_t bi
   return out;
 }
 
-// seq_lens: the sequences' lengths; null: `length` tokens in each.
+// seq_lens: the sequences' lengths; null: `length` tokens in each.  k_new, v_new [B, Hkv, d] of one
+// dtype, on the query's device, contiguous, or null: the token merged into the output (with
+// seq_lens; no lse then).
 std::tuple<at::Tensor, at::Tensor> decode_dl(
     const at::Tensor& q, const at::Tensor& kpairs, const at::Tensor& knorms,
     const at::Tensor& vblocks, const at::Tensor& vnorms, const at::Tensor* seq_lens, int64_t length,
     const at::Tensor& kcentroids, const at::Tensor& vcentroids, const at::Tensor& krotation,
-    const at::Tensor& vrotation, double scale, const c10::optional<at::Tensor>& seq_starts) {
+    const at::Tensor& vrotation, double scale, const c10::optional<at::Tensor>& seq_starts,
+    const at::Tensor* k_new = nullptr, const at::Tensor* v_new = nullptr) {
   require_gpu(q, "q");
   TORCH_CHECK(q.dim() == 3, "q must be [B, Hq, d]");
   TORCH_CHECK(kpairs.dim() == 4 && vblocks.dim() == 4,
@@ -956,7 +959,8 @@ std::tuple<at::Tensor, at::Tensor> decode_dl(
   TORCH_CHECK(kc.numel() == 16 && vc.numel() == (1 << vbits),
               "decode layout: 16 key centroids and 2^vbits value centroids");
   auto out = at::empty({B, Hq, d}, qq.options());
-  auto lse = at::empty({B, Hq}, qq.options().dtype(at::kFloat));
+  at::Tensor lse;
+  if (!k_new) lse = at::empty({B, Hq}, qq.options().dtype(at::kFloat));
   if (B == 0) return {out, lse};
   if (!seq_lens) {
     auto ws = workspace(tq_decode_dl_workspace_bytes((int32_t)B, (int32_t)Hq, (int32_t)Hkv,
@@ -970,6 +974,17 @@ std::tuple<at::Tensor, at::Tensor> decode_dl(
     return {out, lse};
   }
   auto ws = workspace(tq_decode_dl_workspace_bytes((int32_t)B, (int32_t)Hq, (int32_t)Hkv, Tc), dev);
+  if (k_new) {
+    check_rc(tq_decode_attention_dl_merged(
+        qq.data_ptr(), to_tq(qq.scalar_type()), (int32_t)B, (int32_t)Hq, (int32_t)Hkv, (int32_t)d,
+        kpairs.data_ptr<uint8_t>(), knorms.data_ptr(), vblocks.data_ptr<uint8_t>(),
+        vnorms.data_ptr(), to_tq(ndt), Tc, sl.data_ptr<int32_t>(),
+        ss.defined() ? ss.data_ptr<int32_t>() : nullptr, kc.data_ptr<float>(),
+        vc.data_ptr<float>(), Rk.data_ptr<float>(), Rv.data_ptr<float>(), 4, (int32_t)vbits,
+        (float)scale, k_new->data_ptr(), v_new->data_ptr(), to_tq(k_new->scalar_type()),
+        out.data_ptr(), ws.data_ptr(), ws.numel(), cur_stream(qq)));
+    return {out, lse};
+  }
   check_rc(tq_decode_attention_dl_window(
       qq.data_ptr(), to_tq(qq.scalar_type()), (int32_t)B, (int32_t)Hq, (int32_t)Hkv, (int32_t)d,
       kpairs.data_ptr<uint8_t>(), knorms.data_ptr(), vblocks.data_ptr<uint8_t>(),
@@ -1412,13 +1427,22 @@ at::Tensor decode_merge_token(const at::Tensor& o, const at::Tensor& lse, const 
 
 // One decode step of a decode-layout cache in one op: attention over the cached history
 // (decode_attention_dl_lse) merged with the token being decoded, which attends to its own
-// exact key and value (decode_merge_token) -- the same two launches, one dispatch.
+// exact key and value (decode_merge_token): the same result, merged as the output is stored.
 at::Tensor decode_attention_dl_merged(
     const at::Tensor& q, const at::Tensor& kpairs, const at::Tensor& knorms,
     const at::Tensor& vblocks, const at::Tensor& vnorms, const at::Tensor& seq_lens,
     const at::Tensor& kcentroids, const at::Tensor& vcentroids, const at::Tensor& krotation,
     const at::Tensor& vrotation, double scale, const c10::optional<at::Tensor>& seq_starts,
     const at::Tensor& k_new, const at::Tensor& v_new) {
+  if (q.dim() == 3 && kpairs.dim() == 4 && k_new.dim() == 3 && v_new.sizes() == k_new.sizes() &&
+      k_new.size(0) == q.size(0) && k_new.size(1) == kpairs.size(1) && k_new.size(2) == q.size(2)) {
+    require_gpu(q, "q");
+    c10::DeviceGuard g(q.device());
+    auto kn = floatc(k_new, q.device());
+    auto vn = v_new.to(q.device(), kn.scalar_type()).contiguous();
+    return std::get<0>(decode_dl(q, kpairs, knorms, vblocks, vnorms, &seq_lens, -1, kcentroids, vcentroids,
+                                 krotation, vrotation, scale, seq_starts, &kn, &vn));
+  }
   auto ol = decode_attention_dl_lse(q, kpairs, knorms, vblocks, vnorms, seq_lens, kcentroids,
                                     vcentroids, krotation, vrotation, scale, seq_starts);
   return decode_merge_token(std::get<0>(ol), std::get<1>(ol), q, k_new, v_new, scale);

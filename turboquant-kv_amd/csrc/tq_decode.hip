@@ -446,6 +446,37 @@ __global__ __launch_bounds__(kDecThreads, 2) void fused_decode_kernel(DecodeArgs
   }
 }
 
+// The exact current token merged into a decode output by log-sum-exp (the HF cache's
+// rule that the token being decoded attends to its own unquantized key and value,
+// hf_integration.py:372-390): query head `row` of KV head `kvrow`.  s = (q . k_new) * scale;
+// m = max(lse, s); out = (o e^(lse - m) + v_new e^(s - m)) / (e^(lse - m) + e^(s - m)), in
+// fp32, o rounded to the query's type.  The decode kernel (one split) or its combine applies it
+// as it stores; merge_token_kernel to outputs in memory.
+struct NewToken {
+  const void* k;  // [B, hkv, d], null: none
+  const void* v;
+  int dt;
+  float scale;
+};
+// One lane's dims of q . k_new (k_new's and q's loads are the caller's to place early)
+template <int D>
+__device__ __forceinline__ float new_token_dot(const NewToken& t, const void* q, int q_dt, int64_t row, int64_t kvrow) {
+  const int lane = threadIdx.x & 63;
+  float dot = 0.f;
+#pragma unroll
+  for (int j = 0; j < D; j += 64)
+    dot = fmaf(load_as_f32(q, row * D + j + lane, q_dt), load_as_f32(t.k, kvrow * D + j + lane, t.dt), dot);
+  return dot;
+}
+// dot: the wave's sum of new_token_dot; o and v of one dim
+__device__ __forceinline__ float merge_new_token(float dot, float scale, float o, float v, float lh, int q_dt) {
+  const float sn = dot * scale;
+  const float m = fmaxf(lh, sn);
+  const float wh = expf(lh - m), wn = expf(sn - m), den = wh + wn;
+  const float x = round_to(o, q_dt) * wh + v * wn;
+  return x / den;
+}
+
 // One D-thread block per query row (D = head_dim, 64 or 128): log-sum-exp merge of the
 // splits, o = o_rot / L, out = o @ R_v; lse (natural log) = (max + log2 L) * ln 2.
 template <int D = kDim>
@@ -456,7 +487,8 @@ __global__ __launch_bounds__(D) void fused_combine_kernel(const float* __restric
                                                            int64_t t_max, int hq,
                                                            const float* __restrict__ vrot,
                                                            int out_dt, void* __restrict__ out,
-                                                           float* __restrict__ lse) {
+                                                           float* __restrict__ lse, const void* __restrict__ q,
+                                                           int g, NewToken tok) {
   __shared__ float o_s[D];
   const int64_t row = blockIdx.x;
   const int b = (int)(row / hq);
@@ -465,6 +497,11 @@ __global__ __launch_bounds__(D) void fused_combine_kernel(const float* __restric
   float rcol[D];
 #pragma unroll
   for (int k = 0; k < D; ++k) rcol[k] = vrot[k * D + j];
+  float dot = 0.f, vnew = 0.f;
+  if (tok.k) {  // g: query heads per KV head
+    dot = new_token_dot<D>(tok, q, out_dt, row, row / g);
+    vnew = load_as_f32(tok.v, row / g * D + j, tok.dt);
+  }
   // (no seq_lens: every sequence has t_max tokens)
   const int64_t T = seq_lens ? min((int64_t)max(seq_lens[b], 0), t_max) : t_max;
   const int ns = (int)((T + split_tokens - 1) / split_tokens);
@@ -483,8 +520,10 @@ __global__ __launch_bounds__(D) void fused_combine_kernel(const float* __restric
   float r = 0.f;
 #pragma unroll
   for (int k = 0; k < D; ++k) r = fmaf(o_s[k], rcol[k], r);
+  const float lh = any ? (M + log2f(L)) * 0.69314718055994531f : -INFINITY;
+  if (tok.k) r = merge_new_token(wave_sum(dot), tok.scale, r, vnew, lh, out_dt);
   store_from_f32(out, row * D + j, r, out_dt);
-  if (lse && j == 0) lse[row] = any ? (M + log2f(L)) * 0.69314718055994531f : -INFINITY;
+  if (lse && j == 0) lse[row] = lh;
 }
 
 // ------------------------------------------------------------------ decode layout
@@ -547,6 +586,7 @@ struct DlArgs {
   const float* vrot;
   void* out;
   float* lse;
+  NewToken tok;  // merged into the output (contiguous caches)
   // Paged pools (PAGED kernels): block b of a sequence holds its tokens [b*bs, (b+1)*bs);
   // kpairs [num_blocks][hkv][bs][32], knorms/vnorms [num_blocks][hkv][bs], vblocks
   // [num_blocks][hkv][bs/64][1024] for bs a power of two >= 64 (a 64-token tile lies in
@@ -926,7 +966,13 @@ __global__ __launch_bounds__(kDlThreads, 1) void dl_decode_kernel(DlArgs a) {
   // and lse -inf)
   if (SPW == 1 && t_begin >= t_end) {  // uniform
     if (a.out != nullptr && T == 0 && tid < a.G * D) {  // empty sequence: zeros, lse -inf
-      store_from_f32(a.out, qh0 * D + tid, 0.f, a.q_dt);
+      float r = 0.f;
+      if (!PAGED && a.tok.k) {  // whole waves: tid < G D
+        const float dot = wave_sum(new_token_dot<D>(a.tok, a.q, a.q_dt, qh0 + tid / D, bg));
+        r = merge_new_token(dot, a.tok.scale, r, load_as_f32(a.tok.v, (int64_t)bg * D + tid % D, a.tok.dt), -INFINITY,
+                            a.q_dt);
+      }
+      store_from_f32(a.out, qh0 * D + tid, r, a.q_dt);
       if (a.lse && qj == 0) a.lse[qh0 + qh] = -INFINITY;
     }
     return;
@@ -1412,6 +1458,16 @@ __global__ __launch_bounds__(kDlThreads, 1) void dl_decode_kernel(DlArgs a) {
     }
   }
 
+  // The new token's loads ahead of the reduction: waves tid / 64 < 4 SPW NH hold head
+  // (tid / D) % 4 of their stream.
+  // (Batch 64 x 8 KV heads x 4,351 tokens, K4/V3, a layer's step: 36.4 us, against 39.6-40.0 with
+  // the merge a launch of its own, 4.1 us for 2,048 query heads.)
+  const bool merged = !PAGED && a.out != nullptr && a.tok.k != nullptr;
+  float ndot = 0.f, nval = 0.f, lh = -INFINITY;
+  if (merged && tid < 4 * SPW * D && live && ((tid / D) & 3) < a.G) {
+    ndot = new_token_dot<D>(a.tok, a.q, a.q_dt, qh0 + ((tid / D) & 3), bg);
+    nval = load_as_f32(a.tok.v, (int64_t)bg * D + tid % D, a.tok.dt);
+  }
   // ---- reduction: l over the lanes of a head; outputs over the waves (LDS)
   l += __shfl_xor(l, 4);
   l += __shfl_xor(l, 8);
@@ -1460,8 +1516,8 @@ __global__ __launch_bounds__(kDlThreads, 1) void dl_decode_kernel(DlArgs a) {
     } else {  // the whole sequence: out = (o / L) @ R_v here
       qs_s[4 * sw + m][dim] = L > 0.f ? sum / (vsc * L) : 0.f;
     }
-    if (live && a.out != nullptr && m < a.G && dim == 0 && a.lse)
-      a.lse[qh0 + m] = L > 0.f ? (mx[m] + log2f(L)) * 0.69314718055994531f : -INFINITY;
+    lh = L > 0.f ? (mx[m] + log2f(L)) * 0.69314718055994531f : -INFINITY;
+    if (live && a.out != nullptr && m < a.G && dim == 0 && a.lse) a.lse[qh0 + m] = lh;
   }
   if (a.out != nullptr) {
     __syncthreads();
@@ -1476,6 +1532,7 @@ __global__ __launch_bounds__(kDlThreads, 1) void dl_decode_kernel(DlArgs a) {
 #pragma unroll 8
           for (int k = 0; k < D; ++k) r = fmaf(qs_s[4 * sw + m][k], a.vrot[k * D + dim], r);
         }
+        if (merged) r = merge_new_token(wave_sum(ndot), a.tok.scale, r, nval, lh, a.q_dt);
         store_from_f32(a.out, (qh0 + m) * D + dim, r, a.q_dt);
       }
     }
@@ -1915,7 +1972,7 @@ int launch_fused_decode(const FusedDecodeCall& c, void* workspace, size_t worksp
   if (rc != TQ_OK) return rc;
   hipLaunchKernelGGL(fused_combine_kernel<kDim>, dim3((unsigned)rows), dim3(kDim), 0, st, a.part,
                      a.stats, p.nsplit, p.split_tokens, c.seq_lens, c.t_max, c.hq, c.vrot,
-                     c.q_dt, c.out, c.lse);
+                     c.q_dt, c.out, c.lse, nullptr, 1, NewToken{});
   TQ_LAUNCH_CHECK("fused_combine_kernel");
   return TQ_OK;
 }
@@ -2040,11 +2097,7 @@ void launch_dl_paged(int vbits, tq_dtype q_dtype, unsigned grid, const DlArgs& a
   else launch_dl_kernel<PG, 4>(q_dtype, grid, a, st);
 }
 
-// The exact current token merged into a decode output by log-sum-exp (the HF cache's
-// rule that the token being decoded attends to its own unquantized key and value,
-// hf_integration.py:372-390): one wave per query head h of batch row b, KV head
-// h / (hq / hkv).  s = (q . k_new) * scale; m = max(lse, s); out = (o e^(lse - m) +
-// v_new e^(s - m)) / (e^(lse - m) + e^(s - m)), in fp32, stored in the query's type.  `out`
+// The merge of the current token over decode outputs in memory: one wave per query head.  `out`
 // may be `o` (each element is read and then written by the same lane).
 __global__ __launch_bounds__(64) void merge_token_kernel(const void* o, const float* __restrict__ lse,
                                                          const void* __restrict__ q,
@@ -2061,14 +2114,10 @@ __global__ __launch_bounds__(64) void merge_token_kernel(const void* o, const fl
   for (int j = lane; j < d; j += 64)
     dot = fmaf(load_as_f32(q, row * d + j, q_dt), load_as_f32(knew, kvrow * d + j, kv_dt), dot);
   dot = wave_sum(dot);
-  const float sn = dot * scale;
   const float lh = lse[row];
-  const float m = fmaxf(lh, sn);
-  const float wh = expf(lh - m), wn = expf(sn - m), den = wh + wn;
-  for (int j = lane; j < d; j += 64) {
-    const float x = load_as_f32(o, row * d + j, q_dt) * wh + load_as_f32(vnew, kvrow * d + j, kv_dt) * wn;
-    store_from_f32(out, row * d + j, x / den, q_dt);
-  }
+  for (int j = lane; j < d; j += 64)
+    store_from_f32(out, row * d + j, merge_new_token(dot, scale, load_as_f32(o, row * d + j, q_dt),
+                                                     load_as_f32(vnew, kvrow * d + j, kv_dt), lh, q_dt), q_dt);
 }
 
 // The decode-layout kernel over every (stream, split), in launches of at most four query
@@ -2121,11 +2170,11 @@ int run_dl(DlArgs a, tq_dtype q_dtype, int B, int hq, int hkv, int vbits, int pg
   if (d == 128)
     hipLaunchKernelGGL(fused_combine_kernel<128>, dim3((unsigned)rows), dim3(128), 0, st, part, stats,
                        p.nsplit, p.split_tokens, a.seq_lens, a.seq_lens ? a.t_cap : (int64_t)a.len, hq, a.vrot, (int)q_dtype, out,
-                       lse);
+                       lse, a.q, hq / hkv, a.tok);
   else
     hipLaunchKernelGGL(fused_combine_kernel<kDim>, dim3((unsigned)rows), dim3(kDim), 0, st, part, stats,
                        p.nsplit, p.split_tokens, a.seq_lens, a.seq_lens ? a.t_cap : (int64_t)a.len, hq, a.vrot, (int)q_dtype, out,
-                       lse);
+                       lse, a.q, hq / hkv, a.tok);
   TQ_LAUNCH_CHECK("fused_combine_kernel");
   return TQ_OK;
 }
@@ -2146,7 +2195,7 @@ int decode_dl(const void* q, tq_dtype q_dtype, int32_t B, int32_t hq,
               const float* vcentroids, const float* krotation,
               const float* vrotation, int32_t kbits, int32_t vbits,
               float scale, void* out, float* lse, void* workspace,
-              size_t workspace_bytes, void* stream) {
+              size_t workspace_bytes, void* stream, const NewToken* tok = nullptr) {
   TQ_REQUIRE(valid_dtype(q_dtype) && valid_dtype(norm_dtype), "unknown dtype");
   if ((d != 64 && d != 128) || kbits != 4 || vbits < 2 || vbits > 4)
     return fail(TQ_EUNSUPPORTED, "decode layout covers head_dim 64 and 128 with 4-bit keys and "
@@ -2179,6 +2228,7 @@ int decode_dl(const void* q, tq_dtype q_dtype, int32_t B, int32_t hq,
   a.len = seq_lens ? 0 : (int32_t)len;
   a.seq_starts = seq_starts; a.kcen = kcentroids; a.vcen = vcentroids; a.krot = krotation;
   a.vrot = vrotation; a.qscale = scale * 1.4426950408889634f;
+  if (tok) a.tok = *tok;
   return run_dl(a, q_dtype, B, hq, hkv, vbits, 0, p, workspace, out, lse, as_stream(stream),
                 (int)norm_dtype, d);
 }
@@ -2221,6 +2271,24 @@ int tq_decode_attention_dl_len(const void* q, tq_dtype q_dtype, int32_t B, int32
   return decode_dl(q, q_dtype, B, hq, hkv, d, kpairs, knorms, vblocks, vnorms, norm_dtype, t_cap, nullptr, len,
                    nullptr, kcentroids, vcentroids, krotation, vrotation, kbits, vbits, scale, out, lse,
                    workspace, workspace_bytes, stream);
+}
+
+int tq_decode_attention_dl_merged(const void* q, tq_dtype q_dtype, int32_t B, int32_t hq,
+                                  int32_t hkv, int32_t d, const uint8_t* kpairs,
+                                  const void* knorms, const uint8_t* vblocks,
+                                  const void* vnorms, tq_dtype norm_dtype, int64_t t_cap,
+                                  const int32_t* seq_lens, const int32_t* seq_starts,
+                                  const float* kcentroids, const float* vcentroids,
+                                  const float* krotation, const float* vrotation, int32_t kbits,
+                                  int32_t vbits, float scale, const void* k_new, const void* v_new,
+                                  tq_dtype kv_dtype, void* out, void* workspace,
+                                  size_t workspace_bytes, void* stream) {
+  TQ_REQUIRE((seq_lens && k_new && v_new) || B <= 0, "null pointer argument");
+  TQ_REQUIRE(valid_dtype(kv_dtype), "unknown dtype");
+  const NewToken tok{k_new, v_new, (int)kv_dtype, scale};
+  return decode_dl(q, q_dtype, B, hq, hkv, d, kpairs, knorms, vblocks, vnorms, norm_dtype, t_cap, seq_lens, -1,
+                   seq_starts, kcentroids, vcentroids, krotation, vrotation, kbits, vbits, scale, out, nullptr,
+                   workspace, workspace_bytes, stream, &tok);
 }
 
 int tq_decode_attention_dl(const void* q, tq_dtype q_dtype, int32_t B, int32_t hq, int32_t hkv,
