@@ -1,5 +1,5 @@
 """PagedKVPools.forward's prefill rows: written by the kernel in the result's type, equal to
-the fp32 result rounded once, also where the result is a given tensor, an unaligned one or
+the fp32 result converted once, also where the result is a given tensor, an unaligned one or
 the queries' own memory."""
 import pytest
 import torch
@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
 
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32, torch.float64])
 @pytest.mark.parametrize("how", ["none", "given", "unaligned", "alias"])
 def test_forward_prefill_rows(dtype, how):
     from turboquant_kv.vllm_plugin import PagedKVPools, TurboQuantAttentionMetadata
@@ -39,4 +39,4 @@ def test_forward_prefill_rows(dtype, how):
     got = pools.forward(q, k, v, md, 0.125, output=out)
     if out is not None:
         assert got.data_ptr() == out.data_ptr()
-    assert got.dtype == dtype and torch.equal(got, want)  # the same sums, rounded once
+    assert got.dtype == dtype and torch.equal(got, want)  # the same sums, converted once

@@ -346,7 +346,9 @@ class PagedKVPools:
                                   md.seq_lens[:npf].to(torch.int64)]).tolist()
                 qsl, lens = both[:npf + 1], both[npf + 1:]
             # a result that shares the queries' memory takes a sequence's rows after they are read
-            direct = (out.dtype == query.dtype and out.device == query.device == self.kcen.device
+            # (float64 queries are computed in float32, so their result is converted)
+            direct = (out.dtype == query.dtype and query.dtype != torch.float64
+                      and out.device == query.device == self.kcen.device
                       and out.untyped_storage().data_ptr() != query.untyped_storage().data_ptr())
             for i in range(npf):
                 a, b = qsl[i], qsl[i + 1]
