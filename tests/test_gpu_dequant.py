@@ -76,6 +76,24 @@ def test_cache_and_new_tokens(d, vb, dt):
             check(v[:, :, :T], vc.view(B, H, T, d), vno[:, :, :T].float(), vcen, vR, dt)
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d,vb", [(64, 2), (64, 3), (128, 4)])
+def test_cache_norms_wider_than_the_result(d, vb, dt):
+    """fp32 norms of a cache are rounded to a 16-bit result's type before they are multiplied in:
+    the rows of a cache that holds them rounded, bit for bit."""
+    from turboquant_kv._lib import ops as tops
+    g = torch.Generator(device=DEV).manual_seed(d + vb)
+    B, H, cap, T = 2, 3, 128, 100
+    kp = torch.randint(0, 256, (B, H, cap, d // 2), generator=g, device=DEV, dtype=torch.uint8)
+    vp = torch.randint(0, 256, (B, H, cap // 64, 8 * vb * d), generator=g, device=DEV, dtype=torch.uint8)
+    kn, vn = (torch.exp(torch.randn(B, H, cap, generator=g, device=DEV) * 2) for _ in range(2))
+    (_, _, _, kcen, kR), (_, _, _, vcen, vR) = data(d, 4, 1, 1), data(d, vb, 1, 2)
+    got = tops().dequantize_cache_dl(kp, kn, vp, vn, T, kcen, kR, vcen, vR, dt)
+    want = tops().dequantize_cache_dl(kp, kn.to(dt), vp, vn.to(dt), T, kcen, kR, vcen, vR, dt)
+    for a, b in zip(got, want):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
 def test_layer_update_keeps_gradients():
     """A layer's update returns tensors through which new tokens' gradients still flow."""
     from turboquant_kv.config import TurboQuantConfig

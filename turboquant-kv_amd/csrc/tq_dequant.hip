@@ -88,7 +88,9 @@ __device__ __forceinline__ void dequant_side(const DqArgs& a, const DqSide& sd, 
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int64_t tk = t0 + 16 * u + c16;
-      r.n[u] = tk < a.T ? load_as_f32(sd.norms, s * a.t_cap + tk, a.norm_dt) : 0.f;
+      // a cache's fp32 norms are rounded to a 16-bit result's type first; bit-plane rows' are taken as given
+      const float n = tk < a.T ? load_as_f32(sd.norms, s * a.t_cap + tk, a.norm_dt) : 0.f;
+      r.n[u] = SRC == kPlanes ? n : round_to(n, OUT);
       if constexpr (SRC == kKeys) {
         const uint8_t* p = sd.src + (s * a.t_cap + (tk < a.T ? tk : a.T - 1)) * (D / 2) + (D / 8) * g;
 #pragma unroll
