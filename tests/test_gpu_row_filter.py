@@ -33,6 +33,18 @@ def database(N, d, bits, prod, pairs, seed):
     return dict(p=p, sg=sg, rn=rn, nm=nm, cen=cen, R=R, S=S, bits=bits, prod=prod, pairs=pairs, d=d, N=N)
 
 
+def random_rows(N, d, bits, prod, seed):
+    """A database of random codes: any bytes are rows."""
+    from turboquant_kv.codebook import lloyd_max_codebook, make_qjl_matrix, make_rotation_matrix
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    byte = lambda w: torch.randint(0, 256, (N, w), generator=g, device=DEV, dtype=torch.uint8)  # noqa: E731
+    nm = torch.exp(torch.randn(N, generator=g, device=DEV) * 0.3)
+    bpp = (d + 7) // 8
+    return dict(p=byte((bits - prod) * bpp), sg=byte(bpp) if prod else None, rn=nm * 0.3 if prod else None, nm=nm,
+                cen=lloyd_max_codebook(bits - prod, d)[1].to(DEV), R=make_rotation_matrix(d, 42).to(DEV),
+                S=make_qjl_matrix(d, d, 42).to(DEV), bits=bits, prod=prod, pairs=0, d=d, N=N)
+
+
 def scan(db, q, k, filtered):
     Q, N, d, bits = q.shape[0], db["N"], db["d"], db["bits"]
     L, c = capi.lib(), capi
@@ -40,7 +52,7 @@ def scan(db, q, k, filtered):
     small = L.tq_scan_workspace_bytes(c.i64(Q), c.i32(d), c.i32(bits), c.i64(N), c.i32(k))
     big = L.tq_scan_rows_workspace_bytes(c.i64(Q), c.i32(d), c.i32(bits), c.i64(N), c.i32(k),
                                          c.i32(db["prod"]), c.i32(db["pairs"]))
-    ws = torch.empty(big if filtered else small, dtype=torch.uint8, device=DEV)
+    ws = torch.full((big if filtered else small,), 0xab, dtype=torch.uint8, device=DEV)
     s = torch.empty(Q, k, device=DEV)
     i = torch.empty(Q, k, dtype=torch.long, device=DEV)
     dt = {torch.float32: c.TQ_F32, torch.float16: c.TQ_F16, torch.bfloat16: c.TQ_BF16}[q.dtype]
@@ -52,13 +64,15 @@ def scan(db, q, k, filtered):
                   c.p(db["S"]), *tail))
     else:
         c.check(L.tq_ip_scan_topk(*head, c.p(db["nm"]), c.i64(N), c.p(db["cen"]), c.p(db["R"]), *tail))
-    return s, i, big > small
+    # the exact scan writes its lists, at byte 256 of the workspace, for the queries it answers
+    return s, i, big > small, filtered and not bool((ws[256:small] != 0xab).any())
 
 
-def same(db, q, k):
-    s0, i0, _ = scan(db, q, k, False)
-    s1, i1, filters = scan(db, q, k, True)
+def same(db, q, k, unflagged=False):
+    s0, i0, _, _ = scan(db, q, k, False)
+    s1, i1, filters, alone = scan(db, q, k, True)
     assert torch.equal(s0.view(torch.int32), s1.view(torch.int32)) and torch.equal(i0, i1), (db["N"], q.shape, k)
+    assert alone or not unflagged, (db["N"], q.shape, k)
     return filters
 
 
@@ -92,6 +106,13 @@ def test_prod_pair_rows(d, bits):
         g = torch.Generator(device=DEV).manual_seed(bits)
         for Q, k in ((64, 10), (40, 100), (130, 33)):
             assert same(db, torch.randn(Q, d, generator=g, device=DEV).half(), k)
+
+
+@pytest.mark.parametrize("N,k", [(28_000_001, 100), (80_000_001, 32)])
+def test_lists_hold_large_tables(N, k):
+    """The listed rows fit the merge however many rows there are: no query goes on to the exact scan."""
+    db = random_rows(N, 16, 2, 0, k)
+    assert same(db, torch.randn(3, 16, generator=torch.Generator(device=DEV).manual_seed(k), device=DEV), k, True)
 
 
 @pytest.mark.parametrize("prod", [0, 1])

@@ -3805,7 +3805,7 @@ struct RfLayout {
 constexpr int64_t kRfRound = 256;
 
 // Offsets past `base`, where the exact scan's lists lie.
-RfLayout rf_layout(int64_t nq, int d, int64_t N, bool prod, size_t base) {
+RfLayout rf_layout(int64_t nq, int d, int64_t N, int k, bool prod, size_t base) {
   RfLayout L{};
   const int64_t round = std::min(nq, kRfRound);
   L.passes = (int)((round + kRfQ - 1) / kRfQ);
@@ -3815,6 +3815,12 @@ RfLayout rf_layout(int64_t nq, int d, int64_t N, bool prod, size_t base) {
   // a quarter of the rows, 256 to 4,096 groups, in buckets of a group or two: about 4 k rows
   // (more above a million) reach the k-th largest maximum
   L.nsgroups = (int)std::min<int64_t>(ngroups, std::min<int64_t>(4096, std::max<int64_t>(256, ngroups / 4)));
+  // k of the sampled rows reach tau, so about k ngroups / nsgroups of all rows are listed, a little
+  // more for the bounds' width: a third of what the merge holds at most, however large the table
+  // (4,096 groups alone filled the lists from 27M rows at k = 100 on: 30M rows of 100 dims at 2
+    // bits, one query, 1,113 us by the exact scan, 1,702 by the filter and then the exact scan; now 649)
+  const int64_t held = k > kSmallK ? kRfMergeCapBig : kRfMergeCap;
+  L.nsgroups = (int)std::min<int64_t>(ngroups, std::max<int64_t>(L.nsgroups, (3 * k * ngroups + held - 1) / held));
   L.sstride = (int)(ngroups / L.nsgroups);
   L.per_bucket = (L.nsgroups + kRfMaxBuckets - 1) / kRfMaxBuckets;
   L.nbk = (L.nsgroups + L.per_bucket - 1) / L.per_bucket;
@@ -3967,7 +3973,7 @@ size_t tq_scan_rows_workspace_bytes(int64_t nq, int32_t d, int32_t bit_width, in
   const size_t bytes = tq_scan_workspace_bytes(nq, d, bit_width, N, k);
   if (d < 1 || d > 256 || k < 1 || k > kMaxK || !rf_applies(nq, d, N, k, prod ? bit_width - 1 : bit_width, prod, pairs))
     return bytes;
-  return rf_layout(nq, d, N, prod, bytes).total;
+  return rf_layout(nq, d, N, k, prod, bytes).total;
 }
 
 size_t tq_scan_pairs_workspace_bytes(int64_t nq, int32_t d, int64_t N, int32_t k) {
@@ -4041,7 +4047,7 @@ int ip_scan_topk(const void* queries, tq_dtype q_dtype, int64_t nq, int32_t d,
   // (tq_scan_rows_workspace_bytes); the exact scan then answers the queries it flagged.
   int32_t* flag = nullptr;
   if (rf_applies(nq, d, N, k, code_bits, prod != nullptr, pairs) && fast_aligned(a)) {
-    const RfLayout L = rf_layout(nq, d, N, prod != nullptr, need);
+    const RfLayout L = rf_layout(nq, d, N, k, prod != nullptr, need);
     if (workspace_bytes >= L.total && L.nb <= kRfThreads) {
       const int rc = launch_rf(a, code_bits, pairs, static_cast<char*>(workspace), L, &flag, st);
       if (rc != TQ_OK) return rc;
