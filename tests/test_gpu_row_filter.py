@@ -115,6 +115,15 @@ def test_lists_hold_large_tables(N, k):
     assert same(db, torch.randn(3, 16, generator=torch.Generator(device=DEV).manual_seed(k), device=DEV), k, True)
 
 
+@pytest.mark.parametrize("d", [64, 100, 128])
+def test_as_many_results_as_groups(d):
+    """128 results from 128 64-row groups, the least rows that are filtered, and one row more."""
+    for N in (8192, 8193):
+        for bits, prod in ((2, 0), (4, 0), (3, 1)):
+            q = torch.randn(16, d, generator=torch.Generator(device=DEV).manual_seed(d), device=DEV)
+            assert same(database(N, d, bits, prod, 0, d), q, 128, unflagged=True)
+
+
 @pytest.mark.parametrize("prod", [0, 1])
 def test_special_values(prod):
     """Zero, infinite and NaN queries, norms and residual norms, and a database of equal rows: the

@@ -9,7 +9,8 @@
 //   rf_query   q_rot (and S q) per query with the exact scan's sums; fp16 operands scaled by a
 //              power of two per query; beta1, beta2 with
 //                |approx - exact| <= |n| (beta1 + |gamma| beta2) + 2^-100
-//   rf_sample  lower bounds of evenly spaced 64-row groups; per query a bucket's largest
+//   rf_sample  lower bounds of evenly spaced 64-row groups; per query a bucket's largest (a bucket
+//              is 16 rows where there are few groups, else a group or several)
 //   rf_tau     tau = the k-th largest bucket maximum (k distinct rows score at least it)
 //   rf_filter  every row against tau; rf_merge  rescoring and ranking
 // A query with more listed rows than the lists hold is flagged and answered by the exact scan.
@@ -51,6 +52,7 @@ struct RfArgs {
   float* buckets;        // [passes 16][nbk]
   float* tau;            // [passes 16]
   int nbk, per_bucket, sstride, nsgroups, nb;
+  bool fine;             // a bucket per 16 rows (per_bucket 1), else per_bucket groups
   int* cnt;              // [passes][nb][16]
   float* chi;            // [passes][nb][16][kRfCap]
   float* clo;
@@ -377,6 +379,14 @@ __global__ __launch_bounds__(kRfThreads) __attribute__((amdgpu_waves_per_eu(2, 2
   float bmax[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) bmax[r] = -INFINITY;
+  auto store = [&](int at) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float v = row_max16(bmax[r]);
+      if ((lane & 15) == 0) a.buckets[(size_t)(tile * kRfQ + 4 * (lane >> 4) + r) * a.nbk + at] = v;
+      bmax[r] = -INFINITY;
+    }
+  };
   for (int u = 0; u < a.per_bucket; ++u) {
     const int s = bucket * a.per_bucket + u;
     if (s >= a.nsgroups) break;  // uniform
@@ -397,13 +407,10 @@ __global__ __launch_bounds__(kRfThreads) __attribute__((amdgpu_waves_per_eu(2, 2
         const float lo = mid - b;  // no bound from an overflowed one
         if (valid && lo < INFINITY) bmax[r] = fmaxf(bmax[r], lo);
       }
+      if (a.fine) store(4 * bucket + rt);  // uniform
     }
   }
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const float v = row_max16(bmax[r]);
-    if ((lane & 15) == 0 && bucket < a.nbk) a.buckets[(size_t)(tile * kRfQ + 4 * (lane >> 4) + r) * a.nbk + bucket] = v;
-  }
+  if (!a.fine && bucket < a.nbk) store(bucket);
 }
 
 // One block per query: tau = its k-th largest bucket maximum, by bits of an order-preserving key

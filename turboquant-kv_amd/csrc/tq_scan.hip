@@ -3798,6 +3798,7 @@ int launch_mq(const void* queries, tq_dtype q_dtype, int64_t nq, int32_t d, cons
 // ------------------------------------------------------------------ filtered row scan
 struct RfLayout {
   int passes, kt, nsgroups, per_bucket, sstride, nbk, nb;
+  bool fine;
   size_t qrot, qa, qpar, buckets, tau, flag, cnt, chi, clo, cid, total;
 };
 
@@ -3812,18 +3813,23 @@ RfLayout rf_layout(int64_t nq, int d, int64_t N, int k, bool prod, size_t base) 
   const int bpp = (d + 7) / 8, need = (bpp + 3) / 4;
   L.kt = need <= 2 ? 2 : need <= 4 ? 4 : need <= 7 ? 7 : 8;
   const int64_t ngroups = (N + 63) / 64;
-  // a quarter of the rows, 256 to 4,096 groups, in buckets of a group or two: about 4 k rows
+  // a quarter of the rows, 256 to 4,096 groups, in up to 2,048 buckets: about 4 k rows
   // (more above a million) reach the k-th largest maximum
   L.nsgroups = (int)std::min<int64_t>(ngroups, std::min<int64_t>(4096, std::max<int64_t>(256, ngroups / 4)));
   // k of the sampled rows reach tau, so about k ngroups / nsgroups of all rows are listed, a little
   // more for the bounds' width: a third of what the merge holds at most, however large the table
   // (4,096 groups alone filled the lists from 27M rows at k = 100 on: 30M rows of 100 dims at 2
-    // bits, one query, 1,113 us by the exact scan, 1,702 by the filter and then the exact scan; now 649)
+  // bits, one query, 1,113 us by the exact scan, 1,702 by the filter and then the exact scan; now 649)
   const int64_t held = k > kSmallK ? kRfMergeCapBig : kRfMergeCap;
   L.nsgroups = (int)std::min<int64_t>(ngroups, std::max<int64_t>(L.nsgroups, (3 * k * ngroups + held - 1) / held));
   L.sstride = (int)(ngroups / L.nsgroups);
   L.per_bucket = (L.nsgroups + kRfMaxBuckets - 1) / kRfMaxBuckets;
   L.nbk = (L.nsgroups + L.per_bucket - 1) / L.per_bucket;
+  // few groups: a bucket per 16 rows, as k group maxima of not many more bound little (8,192 rows,
+  // k = 128: the smallest of 128 maxima listed every tenth row, which overflowed the lists: 64
+  // dims, 2 bits, 16 queries 285 us by the exact scan, 338 by both)
+  L.fine = L.nsgroups * 4 <= kRfMaxBuckets;
+  if (L.fine) L.nbk = 4 * L.nsgroups;
   L.nb = filter_blocks(N);
   const size_t slots = (size_t)L.passes * L.nb * kRfQ;
   size_t o = align_up(base, 256);
@@ -3867,9 +3873,10 @@ bool rf_applies(int64_t nq, int d, int64_t N, int k, int bits, bool prod, bool p
 template <int BITS, int KT, bool PROD, bool PAIRS>
 int launch_rf_t(const RfArgs& a, const RfLayout& L, hipStream_t st) {
   const unsigned passes = (unsigned)L.passes;
+  const int waves = (L.nsgroups + L.per_bucket - 1) / L.per_bucket;
   hipLaunchKernelGGL((rf_query_kernel<KT, PROD>), dim3(passes * kRfQ), dim3(PROD ? 512 : 256), 0, st, a);
   TQ_LAUNCH_CHECK("rf_query_kernel");
-  hipLaunchKernelGGL((rf_sample_kernel<BITS, KT, PROD, PAIRS>), dim3((unsigned)((L.nbk + kRfWaves - 1) / kRfWaves), passes),
+  hipLaunchKernelGGL((rf_sample_kernel<BITS, KT, PROD, PAIRS>), dim3((unsigned)((waves + kRfWaves - 1) / kRfWaves), passes),
                      dim3(kRfThreads), 0, st, a);
   TQ_LAUNCH_CHECK("rf_sample_kernel");
   hipLaunchKernelGGL(rf_tau_kernel, dim3(passes * kRfQ), dim3(kRfThreads), 0, st, a);
@@ -3927,6 +3934,7 @@ int launch_rf(const ScanArgs& s0, int bits, bool pairs, char* ws, const RfLayout
     a.clo = reinterpret_cast<float*>(ws + L.clo);
     a.cid = reinterpret_cast<int*>(ws + L.cid);
     a.nbk = L.nbk; a.per_bucket = L.per_bucket; a.sstride = L.sstride; a.nsgroups = L.nsgroups; a.nb = L.nb;
+    a.fine = L.fine;
     a.out_s = s.out_s; a.out_i = s.out_i;
     int rc;
     if (s.signs) rc = bits == 2 ? launch_rf_bits<2, true>(a, L, pairs, st) : launch_rf_bits<3, true>(a, L, pairs, st);
