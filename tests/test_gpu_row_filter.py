@@ -124,6 +124,22 @@ def test_as_many_results_as_groups(d):
             assert same(database(N, d, bits, prod, 0, d), q, 128, unflagged=True)
 
 
+@pytest.mark.parametrize("d,bits,N,nq,k", [(128, 4, 1_000_000, 4, 1), (64, 4, 1_000_000, 6, 2), (64, 2, 1_000_000, 4, 1)])
+def test_few_results_around_a_million_rows_scan_exactly(d, bits, N, nq, k):
+    """Calls that the exact scan answers faster ask for its workspace only."""
+    c, L = capi, capi.lib()
+    L.tq_scan_rows_workspace_bytes.restype = ctypes.c_size_t
+    size = lambda n, q, kk, prod=0, pairs=0: L.tq_scan_rows_workspace_bytes(  # noqa: E731
+        c.i64(q), c.i32(d), c.i32(bits), c.i64(n), c.i32(kk), c.i32(prod), c.i32(pairs))
+    base = lambda n, q, kk: L.tq_scan_workspace_bytes(q, d, bits, n, kk)  # noqa: E731
+    assert size(N, nq, k) == base(N, nq, k)
+    assert size(N, nq, 32) > base(N, nq, 32) and size(N // 10, nq, k) > base(N // 10, nq, k)
+    if d == 64 and bits == 4:  # prod pair rows
+        assert size(10_000_000, 2, 10, 1, 1) == base(10_000_000, 2, 10)
+        assert size(10_000_000, 3, 10, 1, 1) == base(10_000_000, 3, 10)
+        assert size(10_000_000, 2, 100, 1, 1) > base(10_000_000, 2, 100)
+
+
 @pytest.mark.parametrize("prod", [0, 1])
 def test_special_values(prod):
     """Zero, infinite and NaN queries, norms and residual norms, and a database of equal rows: the

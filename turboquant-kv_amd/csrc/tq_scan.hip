@@ -3849,24 +3849,43 @@ RfLayout rf_layout(int64_t nq, int d, int64_t N, int k, bool prod, size_t base) 
 }
 
 // Where the filtered row scan answers: bit-plane rows of 2-4 bit codes (prod: 2 or 3) and prod
-// pair rows, 8,192 rows or more (shorter calls are a few steps per wave either way).  Times at
-// k = 10 / 100, exact scan -> filtered, in us:
+// pair rows, 8,192 rows or more (shorter calls are a few steps per wave either way).  Times
+// exact scan -> filtered, in us, at k = 10 / 100 where no k is given:
 //   other dims than 64 and 128 (the exact scan's generic loader): always.  200 dims prod, 390,001
 //     rows: 1 query 125 / 171 -> 100 / 115, 16 queries 717 / 698 -> 101 / 117; 10,000 rows, 1
-//     query 115 / 156 -> 73 / 76; 100 dims, 1M rows, 16 queries 516 / 823 -> 79 / 92
+//     query 115 / 156 -> 73 / 76; 100 dims, 1M rows, 16 queries 516 / 823 -> 79 / 92.  One query
+//     over 2-bit codes without signs, where the exact scan is cheapest: 16 dims, 8,192 rows 57 / 98 ->
+//     36 / 39, 1M 66 -> 49, 80M 2,128 / 2,316 -> 1,051 / 1,080; 160 dims (padded to 224) 8,192
+//     rows 75 / 116 -> 54 / 58, 1M 95 -> 90; 200 dims 1M 103 -> 98, 30M 2,097 -> 898
 //   bit planes of 64 / 128 dims: from 5 queries, 4 up to a million rows, 2 for k > 32.  128 dims
 //     4 bits, 1M rows: 2 queries 79 / 154 -> 107 / 121, 4 queries 104 / 232 -> 108 / 122, 16
-//     queries 281 / 816 -> 108 / 125; 100,000 rows, 4 queries 86 / 196 -> 65 / 81
+//     queries 281 / 816 -> 108 / 125; 100,000 rows, 4 queries 86 / 196 -> 65 / 81.  k up to 4,
+//     whose exact lists cost little, loses around a million rows, where the sample is largest
+//     beside the filter: 4 bits, 4 queries, k = 1, 128 dims 1M 79 -> 101, 300,000 65 -> 67; 64 dims
+//     1M 55 -> 68, 6 queries 61 -> 67 (8: 75 -> 68; 3M, 5: 146 -> 107); 3 bits
+//     1M, 4 queries 53 -> 57
 //   prod pair rows (one exact pass per query): from 2 queries, by the exact scan's work.  128 dims,
 //     1M rows: 2 queries 60 / 101 -> 74 / 90, 4 queries 87 / 138 -> 76 / 91, 16 queries 283 /
 //     372 -> 79 / 92; 10M rows, 1 query 157 -> 253, 2 queries 316 -> 267; 10,000 rows, 64
-//     queries 39 / 70 -> 51 / 54
+//     queries 39 / 70 -> 51 / 54.  At 64 dims two queries need k > 64 (10M rows, 3 bits, k = 10 120
+//     -> 188, k = 64 196 -> 199, k = 128 533 -> 208) and three a few million rows at most (3M 92
+//     -> 83, 10M 171 -> 189).  k = 33 .. 64: 64 dims 1M rows, 3 queries 52 -> 61, 4 queries 70 -> 61;
+//     128 dims 300,000, 4 queries 53 -> 56, 6 queries 78 -> 57
 bool rf_applies(int64_t nq, int d, int64_t N, int k, int bits, bool prod, bool pairs) {
   if (nq < 1 || nq > INT_MAX || N < 8192 || bits < 2 || bits > (prod ? 3 : 4) || d < 16) return false;
   const int bpp = (d + 7) / 8;
-  if (pairs) return prod && nq >= 2 && (double)N * nq * d >= (k > kSmallK ? 1.2e8 : 4e8);
+  if (pairs) {
+    if (!prod || nq < 2) return false;
+    if (d == 64 && nq == 2 && k <= 64) return false;
+    if (d == 64 && nq == 3 && k < kSmallK && N > 5000000) return false;
+    return (double)N * nq * d >= (k <= kSmallK ? 4e8 : k <= 64 && nq <= 5 ? 2e8 : 1.2e8);
+  }
   if (bpp != 8 && bpp != 16) return true;
   if (k > kSmallK) return nq >= 2;
+  if (k <= 4 && N > 250000 && N < 2000000) {
+    if (k <= 2 && bits == 4 && bpp == 8) return nq >= 7;
+    if (nq == 4 && (bits == 4 || (k <= 2 && bpp == 8))) return N <= 500000;
+  }
   return nq >= 5 || (nq == 4 && N <= 1000000);
 }
 
