@@ -2043,23 +2043,29 @@ def test_prod_scan_rejects_bad_bits():
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
 def test_quantize_few_rows_equals_tiled_kernel(d, dt):
-    """A call of at most 16384 bf16/fp16 rows of d 64/128 (a decode step's append) runs one
-    wave per row; its codes and norms equal the tiled kernel's -- the same rows inside a
-    call of 20,000 rows -- bit for bit, and the oracle's outside the decision band."""
+    """A few bf16/fp16 rows of d 64/128: on the matrix cores where they are 16-byte aligned, a
+    wave per row (up to 16384) where they are not or round in another type; codes and norms
+    equal the tiled kernel's -- the same rows inside an unaligned call of 20,000 rows -- bit
+    for bit, and the oracle's outside the decision band."""
     g = torch.Generator(device=DEV).manual_seed(d)
     x = torch.randn(20000, d, generator=g, device=DEV) * 3
     x[5] = 0.0
     tdt = torch.bfloat16 if dt == "bf16" else torch.float16
     cdt = capi.TQ_BF16 if dt == "bf16" else capi.TQ_F16
     xt = x.to(tdt).contiguous()
+    odd = lambda t: torch.empty(t.numel() + 1, dtype=tdt, device=DEV)[1:].view(t.shape).copy_(t)  # noqa: E731
     R = O.dense_qr_rotation(d, 42)
     for bits in (1, 2, 3, 4):
         bnd, _ = O.lloyd_max_codebook(bits, d)
-        big_p, big_n = k_quantize(xt, R, bnd, bits, cdt, cdt)
-        for n in (1, 37, 512):
-            p, nm = k_quantize(xt[:n].contiguous(), R, bnd, bits, cdt, cdt)
-            assert np.array_equal(p, big_p[:n]), (bits, n)
-            assert np.array_equal(nm.view(np.uint32), big_n[:n].view(np.uint32)), (bits, n)
+        big_p, big_n = k_quantize(odd(xt), R, bnd, bits, cdt, cdt)
+        mixed_p, mixed_n = k_quantize(xt, R, bnd, bits, cdt, capi.TQ_F32)
+        for n in (1, 37, 16384, 512):
+            for rows, rdt, want_p, want_n in ((odd(xt[:n]), cdt, big_p, big_n),
+                                              (xt[:n].contiguous(), capi.TQ_F32, mixed_p, mixed_n),
+                                              (xt[:n].contiguous(), cdt, big_p, big_n)):
+                p, nm = k_quantize(rows, R, bnd, bits, cdt, rdt)
+                assert np.array_equal(p, want_p[:n]), (bits, n, rdt)
+                assert np.array_equal(nm.view(np.uint32), want_n[:n].view(np.uint32)), (bits, n, rdt)
         # against the oracle: identical outside the decision band (inside it the reduced-
         # precision sums flip often -- the tiled kernel these equal is the one pinned to
         # reference.py's own bf16 codes by the golden test above)

@@ -1,5 +1,5 @@
-"""The matrix-core quantizer of bf16 / fp16 rows (csrc/tq_q16.h) against the general kernel,
-which rows at an odd 2-byte offset still take: codes and norms bit for bit, since the
+"""The matrix-core quantizer of bf16 / fp16 rows (csrc/tq_q16.h) against the general kernels (a
+wave per row up to 16,384 rows, tiled above), which rows at an odd 2-byte offset take: codes and norms bit for bit, since the
 coordinates whose code its sums leave open are summed again in the general kernel's order.
 """
 
