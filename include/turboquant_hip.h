@@ -61,7 +61,7 @@ int tq_rotate_and_quantize(const void* vectors, tq_dtype in_dtype, tq_dtype roun
 /*
  * tq_rotate_and_quantize of bf16 / fp16 rows (dtype, also the rounding type) of d = 64 or
  * 128: the same codes and norms, the norms [n] in norm_dtype (TQ_F32 or dtype), as a
- * 16-bit model's cache keeps them.  vectors 16-byte aligned.
+ * 16-bit model's cache keeps them.  vectors and rotation 16-byte aligned.
  */
 int tq_quantize_mse_rows(const void* vectors, tq_dtype dtype, int64_t n, int32_t d,
                          const float* rotation, const float* boundaries, int32_t bit_width,

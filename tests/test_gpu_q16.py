@@ -82,3 +82,19 @@ def test_packed_rows_at_any_address(d):
             got.append(buf[off: off + 333 * bits * d // 8].cpu().numpy())
             assert not buf[off + 333 * bits * d // 8:].any()
         assert np.array_equal(got[0], got[1]), bits
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d", [64, 128])
+def test_rotation_at_any_address(d, dt):
+    """A rotation that is not 16-byte aligned goes to the general kernels, few rows and many."""
+    from turboquant_kv._lib import ops
+    from turboquant_kv.codebook import lloyd_max_codebook, make_rotation_matrix
+
+    R = make_rotation_matrix(d, 42).to(DEV)
+    bnd = lloyd_max_codebook(4, d)[0].to(DEV)
+    for n in (1, 300, 16_385):
+        x = rows(n, d, "normal", dt, n)
+        p0, n0 = ops().quantize_mse_packed(x, R, bnd, 4)
+        p1, n1 = ops().quantize_mse_packed(x, unaligned(R), bnd, 4)
+        assert torch.equal(p0, p1) and torch.equal(n0.view(torch.int16), n1.view(torch.int16)), n

@@ -140,6 +140,19 @@ def test_few_results_around_a_million_rows_scan_exactly(d, bits, N, nq, k):
         assert size(10_000_000, 2, 100, 1, 1) > base(10_000_000, 2, 100)
 
 
+def test_matrices_at_any_address():
+    """A rotation and QJL matrix that are not 16-byte aligned."""
+    db = database(9000, 100, 4, 1, 0, 5)
+    q = torch.randn(5, 100, generator=torch.Generator(device=DEV).manual_seed(6), device=DEV)
+    s0, i0, _, _ = scan(db, q, 10, True)
+    for key, off in (("R", 1), ("S", 3)):
+        m = db[key]
+        db[key] = torch.empty(m.numel() + off, device=DEV)[off:].view(m.shape).copy_(m)
+    assert same(db, q, 10, unflagged=True)
+    s1, i1, _, _ = scan(db, q, 10, True)
+    assert torch.equal(s0, s1) and torch.equal(i0, i1)
+
+
 @pytest.mark.parametrize("prod", [0, 1])
 def test_special_values(prod):
     """Zero, infinite and NaN queries, norms and residual norms, and a database of equal rows: the

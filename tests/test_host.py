@@ -84,6 +84,12 @@ def test_capi_rejects_bad_arguments_without_launching():
                                         z, z, z, z, capi.i64(8), z, z, z, z, z, capi.i32(4),
                                         capi.i32(2), ctypes.c_float(1.0), z, z, z, ctypes.c_size_t(0), z)
     assert rc == 1 and b"multiple" in lib.tq_last_error()
+    # kernels that read whole rows and matrices 16 bytes at a time (addresses only: nothing is read)
+    at = lambda v: ctypes.c_void_p(v)  # noqa: E731
+    for rows, rot in ((0x1002, 0x2000), (0x1000, 0x2004)):
+        rc = lib.tq_quantize_mse_rows(at(rows), 2, capi.i64(4), capi.i32(64), at(rot), at(0x3000), capi.i32(4),
+                                      at(0x4000), at(0x5000), 2, z)
+        assert rc == 1 and b"16-byte aligned" in lib.tq_last_error(), (rows, rot)
     # empty inputs are valid no-ops
     assert lib.tq_rotate_and_quantize(z, 0, 0, capi.i64(0), capi.i32(64), z, z, capi.i32(4), z, z, z) == 0
 

@@ -208,7 +208,8 @@ std::tuple<at::Tensor, at::Tensor> quantize_mse_packed(const at::Tensor& vectors
   TORCH_CHECK(bit_width >= 1 && bit_width <= 4, "bit_width must be 1-4");
   TORCH_CHECK(bnd.numel() == (1 << bit_width) - 1, "boundaries length must be 2^bit_width - 1");
   auto packed = at::empty({n, packed_width(bit_width, d)}, x.options().dtype(at::kByte));
-  if (dt != TQ_F32 && (d == 64 || d == 128) && (reinterpret_cast<uintptr_t>(x.data_ptr()) & 15) == 0) {
+  if (dt != TQ_F32 && (d == 64 || d == 128) &&
+      ((reinterpret_cast<uintptr_t>(x.data_ptr()) | reinterpret_cast<uintptr_t>(R.data_ptr())) & 15) == 0) {
     auto nm = at::empty({n}, x.options());  // the kernel writes the norms in the rows' type
     check_rc(tq_quantize_mse_rows(x.data_ptr(), dt, n, (int32_t)d, R.data_ptr<float>(), bnd.data_ptr<float>(),
                                   (int32_t)bit_width, packed.data_ptr<uint8_t>(), nm.data_ptr(), dt,

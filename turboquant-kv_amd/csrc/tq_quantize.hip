@@ -727,7 +727,7 @@ __global__ __launch_bounds__(kThreads) void dequant_kernel(DequantArgs a) {
 // ---------------------------------------------------------------- one row per wave (few rows)
 // quantize_kernel<false>'s arithmetic, bit for bit, for the few bf16/fp16 rows of d = 64 / 128
 // that the matrix-core kernel below does not take (rounding in another type than the rows',
-// rows at an odd address), with one wave per row (lane j owns output dims j and
+// rows or a rotation at an odd address), with one wave per row (lane j owns output dims j and
 // j + 64): 16-row tiles would spread a few hundred rows over a few dozen workgroups, each
 // walking its tile through five barriers (256 rows of 128 dims, 4 bits, rounded in fp32: 20.6
 // us tiled, 12.6 here; unaligned bf16 31.9 / 18.8; 16,384 rows of 64 dims 14.7 / 12.3).  Here R
@@ -903,9 +903,9 @@ __global__ __launch_bounds__(64 * q16::waves<D>(), 4) void quantize16_kernel(Q16
   }
 }
 
-bool use_q16(const void* x, tq_dtype in_dt, tq_dtype rdt, int d) {
+bool use_q16(const void* x, tq_dtype in_dt, tq_dtype rdt, int d, const float* rot) {  // both are read 16 bytes at a time
   return in_dt != TQ_F32 && in_dt == rdt && (d == 64 || d == 128) &&
-         (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
+         ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(rot)) & 15u) == 0;
 }
 
 void launch_q16(const Q16Args& a, int d, tq_dtype dt, hipStream_t st) {
@@ -1015,7 +1015,7 @@ int tq_rotate_and_quantize(const void* vectors, tq_dtype in_dtype, tq_dtype roun
     TQ_LAUNCH_CHECK("quantize_mfma_kernel<mse>");
     return TQ_OK;
   }
-  if (use_q16(vectors, in_dtype, round_dtype, d))
+  if (use_q16(vectors, in_dtype, round_dtype, d, rotation))
     return tq_quantize_mse_rows(vectors, in_dtype, n, d, rotation, boundaries, bit_width, packed, norms, TQ_F32,
                                 stream);
   if ((d == 64 || d == 128) && in_dtype != TQ_F32 && n <= kQrMaxRows) {  // few rows: a wave each
@@ -1044,7 +1044,7 @@ int tq_quantize_mse_rows(const void* vectors, tq_dtype dtype, int64_t n, int32_t
   TQ_REQUIRE(norm_dtype == dtype || norm_dtype == TQ_F32, "norms are float32 or the rows' type");
   if (n == 0) return TQ_OK;
   TQ_REQUIRE(vectors && rotation && boundaries && packed && norms, "null pointer argument");
-  TQ_REQUIRE(use_q16(vectors, dtype, dtype, d), "rows must be 16-byte aligned");
+  TQ_REQUIRE(use_q16(vectors, dtype, dtype, d, rotation), "rows and rotation must be 16-byte aligned");
   launch_q16(Q16Args{static_cast<const uint16_t*>(vectors), n, rotation, boundaries, bit_width, packed, norms,
                      (int)norm_dtype},
              d, dtype, as_stream(stream));

@@ -76,7 +76,7 @@ __global__ __launch_bounds__(PROD ? 512 : 256) void rf_query_kernel(RfArgs a) {
   const int qi = blockIdx.x, mi = threadIdx.x >> 8, j = threadIdx.x & 255, d = a.d;
   const bool real = qi < a.nq;
   const float* __restrict__ mat = mi ? a.qjl : a.rot;
-  const bool wide = (d & 3) == 0;
+  const bool wide = (d & 3) == 0 && (reinterpret_cast<uintptr_t>(mat) & 15u) == 0;
   const int nch = real ? (d + C - 1) / C : 0;  // uniform
   // thread j's pieces of a chunk: row r = 16 i + j / 16, columns 4 (j % 16) ..
   struct Chunk {
