@@ -59,8 +59,6 @@ def test_cache_append(d, vb, dt):
 def test_paged_write(block, vb, dt):
     """Slots of prompts (runs from any offset, several sequences in a batch), of decode tokens
     (scattered), padding and out-of-pool slots; pools keep their other tokens."""
-    from turboquant_kv import ops
-    from turboquant_kv._lib import ops as tops
     H, nb = 3, 40
     Rk, bk, Rv, bv = tables(64, vb)
     g = torch.Generator(device=DEV).manual_seed(block + vb)
@@ -73,19 +71,42 @@ def test_paged_write(block, vb, dt):
              torch.cat([pad, run(48, 64)]), run(0, 32).flip(0),
              torch.cat([run(0, 8), run(24, 24)]), torch.cat([run(3, 13), pad[:1], run(64, 64)])]
     for i, slots in enumerate(cases):
-        n = slots.numel()
-        k, v = (torch.randn(n, H, 64, generator=g, device=DEV).to(dt) for _ in range(2))
-        kp = torch.randint(0, 256, (nb, H, block, 32), generator=g, device=DEV, dtype=torch.uint8)
-        shape = (nb, H, block // 64, 512 * vb) if block >= 64 else (nb, H, block // 16, 128 * vb)
-        vt = torch.randint(0, 256, shape, generator=g, device=DEV, dtype=torch.uint8)
-        kn, vn = (torch.randn(nb, H, block, generator=g, device=DEV) for _ in range(2))
-        want = [t.clone() for t in (kp, kn, vt, vn)]
-        kq, knew = tops().quantize_mse_packed(k.reshape(-1, 64), Rk, bk, 4)
-        vq, vnew = tops().quantize_mse_packed(v.reshape(-1, 64), Rv, bv, vb)
-        pairs = torch.empty(n * H, 1, 32, dtype=torch.uint8, device=DEV)
-        ops.pack_decode_layout(kq.view(n * H, 1, -1), pairs, 64, 4, False, 0)
-        ops.paged_store(pairs.view(n, H, -1), knew.float().view(n, H), slots, want[0], want[1])
-        ops.paged_store_value_tiles(vq.view(n, H, -1), vnew.float().view(n, H), slots, want[2], want[3])
-        tops().paged_write_dl(k, v, slots, kp, kn, vt, vn, Rk, bk, Rv, bv)
-        for got, w, name in zip((kp, kn, vt, vn), want, ("keys", "key norms", "values", "value norms")):
-            assert torch.equal(got, w), (name, i)
+        paged_write_equals_separate_ops(slots, block, vb, dt, H, nb, (Rk, bk, Rv, bv), g, i)
+
+
+@pytest.mark.parametrize("block,vb", [(16, 3), (32, 4), (64, 2), (64, 3), (64, 4), (128, 3)])
+def test_paged_write_large_batches(block, vb):
+    """Hundreds of prompts of ragged lengths, more windows of 16 tokens than the launch has waves:
+    whole sub-blocks beside single tokens that share their value words, in every half."""
+    H, nb, dt = 8, 16384 // block, torch.bfloat16
+    g = torch.Generator(device=DEV).manual_seed(block + vb)
+    lens = torch.randint(17, 63, (256,), generator=g, device=DEV).tolist()
+    starts = torch.randint(0, 40, (256,), generator=g, device=DEV).tolist()
+    # 64 slots a sequence, its new tokens from any offset; every fourth one starts anew
+    slots = torch.cat([torch.arange(n, device=DEV) + 64 * i + min(a if i % 4 else 0, 64 - n)
+                       for i, (n, a) in enumerate(zip(lens, starts))])
+    assert slots.numel() // 16 * H > 4096 and slots.unique().numel() == slots.numel()
+    paged_write_equals_separate_ops(slots, block, vb, dt, H, nb, tables(64, vb), g, "ragged")
+    paged_write_equals_separate_ops(torch.arange(16384, device=DEV), block, vb, dt, H, nb, tables(64, vb), g, "whole")
+
+
+def paged_write_equals_separate_ops(slots, block, vb, dt, H, nb, tab, g, name):
+    from turboquant_kv import ops
+    from turboquant_kv._lib import ops as tops
+    Rk, bk, Rv, bv = tab
+    n = slots.numel()
+    k, v = (torch.randn(n, H, 64, generator=g, device=DEV).to(dt) for _ in range(2))
+    kp = torch.randint(0, 256, (nb, H, block, 32), generator=g, device=DEV, dtype=torch.uint8)
+    shape = (nb, H, block // 64, 512 * vb) if block >= 64 else (nb, H, block // 16, 128 * vb)
+    vt = torch.randint(0, 256, shape, generator=g, device=DEV, dtype=torch.uint8)
+    kn, vn = (torch.randn(nb, H, block, generator=g, device=DEV) for _ in range(2))
+    want = [t.clone() for t in (kp, kn, vt, vn)]
+    kq, knew = tops().quantize_mse_packed(k.reshape(-1, 64), Rk, bk, 4)
+    vq, vnew = tops().quantize_mse_packed(v.reshape(-1, 64), Rv, bv, vb)
+    pairs = torch.empty(n * H, 1, 32, dtype=torch.uint8, device=DEV)
+    ops.pack_decode_layout(kq.view(n * H, 1, -1), pairs, 64, 4, False, 0)
+    ops.paged_store(pairs.view(n, H, -1), knew.float().view(n, H), slots, want[0], want[1])
+    ops.paged_store_value_tiles(vq.view(n, H, -1), vnew.float().view(n, H), slots, want[2], want[3])
+    tops().paged_write_dl(k, v, slots, kp, kn, vt, vn, Rk, bk, Rv, bv)
+    for got, w, what in zip((kp, kn, vt, vn), want, ("keys", "key norms", "values", "value norms")):
+        assert torch.equal(got, w), (what, name)

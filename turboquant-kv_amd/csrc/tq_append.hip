@@ -89,11 +89,24 @@ __device__ __forceinline__ uint32_t share_of(const Share<VB>& o, int j) {
   return VB == 2 ? o.s[0] : (o.s[j >> 1] >> (16 * (j & 1))) & 0xffffu;
 }
 
+// Merges a 16-bit share at byte offset `off` into its word while the word's other half may be
+// written the same way by another wave: whole-word atomics, the bits outside `mask` untouched.
+__device__ __forceinline__ void merge_share(uint8_t* base, int off, uint32_t mask, uint32_t bits) {
+  uint32_t* q = reinterpret_cast<uint32_t*>(base + (off & ~3));
+  const int sh = 8 * (off & 2);
+  atomicAnd(q, ~(mask << sh));
+  atomicOr(q, bits << sh);
+}
+
 // Stores a 16-token sub-block's words of half h: row c16 is token c16 of the sub-block (live
 // or not), m its number in the 64-token tile.  `base`: the tile's half, or the sub-block.
+// In a tile, words of 3 and 4 bits hold two sub-blocks, a 16-bit share each.  `atomic`: single
+// tokens of the other one may be merged (whole-word atomics) meanwhile; a plain 16-bit store
+// would race with those on the word, so the share is merged like them.  Else the other
+// sub-block is not written by this launch, or by plain 16-bit stores to its own bytes.
 template <int VB, bool SUB, int CT>
 __device__ __forceinline__ void store_sub_block(const uint32_t (&code)[CT], int h, bool live, int m,
-                                                uint8_t* base) {
+                                                uint8_t* base, bool atomic = false) {
   const int lane = threadIdx.x & 63, g = lane >> 4, sl = (lane & 15) >> 2, t = lane & 3;
   Share<VB> mask = field_mask<VB>(t), mine{};
   constexpr int NS = VB == 2 ? 1 : 2;
@@ -116,6 +129,12 @@ __device__ __forceinline__ void store_sub_block(const uint32_t (&code)[CT], int 
   for (int j = 0; j < (VB == 2 ? 1 : VB); ++j) {
     const uint32_t mk = share_of<VB>(mask, j), v = share_of<VB>(mine, j);
     if (mk == 0) continue;
+    if constexpr (VB != 2 && !SUB) {
+      if (atomic) {
+        merge_share(base, share_off<VB, SUB>(L, m, j), mk, v);
+        continue;
+      }
+    }
     uint8_t* p = base + share_off<VB, SUB>(L, m, j);
     if constexpr (VB == 2) {
       uint32_t* q = reinterpret_cast<uint32_t*>(p);
@@ -146,12 +165,9 @@ __device__ __forceinline__ void store_token(const uint32_t (&code)[CT], int h, i
     for (int r = 0; r < 4; ++r)
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
-        const int off = share_off<VB, SUB>(16 * sl + 4 * g + r, m, j), sh = 8 * (off & 2);
-        uint32_t* q = reinterpret_cast<uint32_t*>(base + (off & ~3));
-        const uint32_t mk = share_of<VB>(mask, j) << sh;
+        const uint32_t mk = share_of<VB>(mask, j);
         if (mk == 0) continue;
-        atomicAnd(q, ~mk);
-        atomicOr(q, share_of<VB>(o[r], j) << sh);
+        merge_share(base, share_off<VB, SUB>(16 * sl + 4 * g + r, m, j), mk, share_of<VB>(o[r], j));
       }
   } else {
     uint32_t old[4][NJ];
@@ -393,7 +409,8 @@ struct PagedArgs {
 // Window w of 16 new tokens of one head.  Tokens that fill a 16-aligned run of slots (a prompt's
 // body) are taken as whole sub-blocks: the run that holds the window's first token, shifted
 // back to the run's start, when all of its 16 tokens are in the batch; the window before
-// leaves those tokens out.  The window's remaining tokens are merged one by one.
+// leaves those tokens out.  The window's remaining tokens are merged one by one.  A batch names
+// a slot once: the tokens of a whole run are the only ones of its sub-block.
 template <bool BF, bool KEYS, int VB, bool SUB>
 __device__ __forceinline__ void paged_side(const PagedArgs& a, q16::Lds<64>& t, q16::WaveLds<64>* wl) {
   using Q = q16::Quantizer<64, BF, KEYS>;
@@ -417,6 +434,14 @@ __device__ __forceinline__ void paged_side(const PagedArgs& a, q16::Lds<64>& t, 
     const int64_t s = in ? a.slots[b + c16] : -1;
     return __all(in && s == (s0 & ~(int64_t)15) + c16 && s < a.num_slots) ? b : -1;
   };
+  // whether the other sub-block of run b's value words is a whole run of this batch, too (then
+  // its window takes it as one and no single token of it is merged)
+  auto paired = [&](int64_t b) {
+    const int64_t s0 = a.slots[b], o = (s0 & 16) ? b - 16 : b + 16;
+    const bool in = o >= 0 && o + 16 <= a.n;
+    const int64_t s = in ? a.slots[o + c16] : -1;
+    return (bool)__all(in && s == (s0 ^ 16) + c16);
+  };
   auto block_of = [&](int64_t slot, int h) { return ((slot >> a.bs_log2) * a.heads + h) << a.bs_log2; };
   for (; task < tasks; task += step) {
     const int64_t w = task / a.heads;
@@ -439,7 +464,9 @@ __device__ __forceinline__ void paged_side(const PagedArgs& a, q16::Lds<64>& t, 
         if (live) store_key<64>(code, a.pool[SD] + row * 32);
       } else {
         uint8_t* base = a.pool[SD] + (SUB ? (row >> 4) * (128 * VB) : (row >> 6) * (512 * VB));
-        if (pass == 0) store_sub_block<VB, SUB>(code, 0, true, (int)(row >> 4) & 3, base);
+        if (pass == 0) {
+          store_sub_block<VB, SUB>(code, 0, true, (int)(row >> 4) & 3, base, !SUB && VB != 2 && !paired(run));
+        }
         else if (live) store_token<VB, SUB, true>(code, 0, (int)(row & 63), base);
       }
     }
