@@ -22,36 +22,58 @@ def tables(d, vb):
 def test_cache_append(d, vb, dt):
     """Positions and lengths around the 16-token sub-blocks and 64-token tiles, one token per
     stream included; contiguous, transposed and unaligned rows; norms in both types."""
+    g = torch.Generator(device=DEV).manual_seed(10 * d + vb)
+    for pos, n in ((0, 1), (63, 1), (38, 1), (0, 16), (5, 3), (15, 2), (16, 48), (7, 130), (0, 256), (61, 65)):
+        for form in ("contiguous", "transposed", "odd"):
+            append_equals_separate_ops(3, 7, 256, pos, n, d, vb, dt, form, g)
+
+
+@pytest.mark.parametrize("d,vb", [(64, 2), (64, 3), (64, 4), (128, 2), (128, 3), (128, 4)])
+def test_cache_append_large(d, vb):
+    """More 16-token sub-blocks than the launch has waves, from an odd position; one token of more
+    streams than its waves take at once."""
+    g = torch.Generator(device=DEV).manual_seed(10 * d + vb)
+    append_equals_separate_ops(8, 8, 1088, 37, 1000, d, vb, torch.bfloat16, "transposed", g)
+    append_equals_separate_ops(5000, 7, 64, 37, 1, d, vb, torch.bfloat16, "contiguous", g)
+
+
+@pytest.mark.parametrize("d,vb", [(64, 3), (128, 2), (128, 3), (128, 4)])
+def test_cache_append_rotation_at_any_address(d, vb):
+    """Rotations that are not 16-byte aligned: one token a stream and several."""
+    g = torch.Generator(device=DEV).manual_seed(d + vb)
+    for pos, n in ((38, 1), (5, 40)):
+        append_equals_separate_ops(3, 7, 256, pos, n, d, vb, torch.bfloat16, "contiguous", g, odd_rotations=True)
+
+
+def append_equals_separate_ops(B, H, cap, pos, n, d, vb, dt, form, g, odd_rotations=False):
     from turboquant_kv import ops
     from turboquant_kv._lib import ops as tops
     Rk, bk, Rv, bv = tables(d, vb)
-    g = torch.Generator(device=DEV).manual_seed(10 * d + vb)
-    cap, B, H = 256, 3, 7
-    for pos, n in ((0, 1), (63, 1), (38, 1), (0, 16), (5, 3), (15, 2), (16, 48), (7, 130), (0, 256), (61, 65)):
-        for form in ("contiguous", "transposed", "odd"):
-            nd = torch.float32 if form == "transposed" else dt
-            new = lambda *s: torch.randint(0, 256, s, generator=g, device=DEV, dtype=torch.uint8)  # noqa: E731
-            kp, vp = new(B, H, cap, d // 2), new(B, H, cap // 64, 8 * vb * d)
-            kn, vn = (torch.randn(B, H, cap, generator=g, device=DEV).to(nd) for _ in range(2))
-            kv = []
-            for _ in range(2):
-                x = torch.randn(B, n, H, d, generator=g, device=DEV).to(dt)
-                x = x.transpose(1, 2)
-                if form == "contiguous":
-                    x = x.contiguous()
-                elif form == "odd":
-                    buf = torch.empty(x.numel() + 1, dtype=dt, device=DEV)[1:].view(B, H, n, d)
-                    x = buf.copy_(x)
-                kv.append(x)
-            want = [t.clone() for t in (kp, kn, vp, vn)]
-            for x, R, b, c, nm, bits, val in ((kv[0], Rk, bk, want[0], want[1], 4, False),
-                                              (kv[1], Rv, bv, want[2], want[3], vb, True)):
-                p, norms = tops().quantize_mse_packed(x.reshape(-1, d), R, b, bits)
-                ops.pack_decode_layout(p.view(B * H, n, -1), c.view(B * H, c.shape[2], -1), d, bits, val, pos)
-                nm[:, :, pos:pos + n] = norms.view(B, H, n).to(nd)
-            tops().cache_append_dl(kv[0], kv[1], kp, kn, vp, vn, pos, Rk, bk, Rv, bv, 4, vb)
-            for got, w, name in zip((kp, kn, vp, vn), want, ("keys", "key norms", "values", "value norms")):
-                assert torch.equal(got, w), (name, pos, n, form)
+    nd = torch.float32 if form == "transposed" else dt
+    new = lambda *s: torch.randint(0, 256, s, generator=g, device=DEV, dtype=torch.uint8)  # noqa: E731
+    kp, vp = new(B, H, cap, d // 2), new(B, H, cap // 64, 8 * vb * d)
+    kn, vn = (torch.randn(B, H, cap, generator=g, device=DEV).to(nd) for _ in range(2))
+    kv = []
+    for _ in range(2):
+        x = torch.randn(B, n, H, d, generator=g, device=DEV).to(dt)
+        x = x.transpose(1, 2)
+        if form == "contiguous":
+            x = x.contiguous()
+        elif form == "odd":
+            buf = torch.empty(x.numel() + 1, dtype=dt, device=DEV)[1:].view(B, H, n, d)
+            x = buf.copy_(x)
+        kv.append(x)
+    want = [t.clone() for t in (kp, kn, vp, vn)]
+    for x, R, b, c, nm, bits, val in ((kv[0], Rk, bk, want[0], want[1], 4, False),
+                                      (kv[1], Rv, bv, want[2], want[3], vb, True)):
+        p, norms = tops().quantize_mse_packed(x.reshape(-1, d), R, b, bits)
+        ops.pack_decode_layout(p.view(B * H, n, -1), c.view(B * H, c.shape[2], -1), d, bits, val, pos)
+        nm[:, :, pos:pos + n] = norms.view(B, H, n).to(nd)
+    if odd_rotations:
+        Rk, Rv = (torch.empty(R.numel() + 1, device=DEV)[1:].view(d, d).copy_(R) for R in (Rk, Rv))
+    tops().cache_append_dl(kv[0], kv[1], kp, kn, vp, vn, pos, Rk, bk, Rv, bv, 4, vb)
+    for got, w, name in zip((kp, kn, vp, vn), want, ("keys", "key norms", "values", "value norms")):
+        assert torch.equal(got, w), (name, pos, n, form)
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])

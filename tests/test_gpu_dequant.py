@@ -39,10 +39,11 @@ def data(d, bits, n, seed):
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("d", [64, 128])
 def test_bitplane_rows(d, dt):
-    """1-4 bits, row counts around the 32-token steps and the workgroups."""
+    """1-4 bits, row counts around the 32-token steps and the workgroups, and more rows than the
+    launch's waves take in one step."""
     from turboquant_kv._lib import ops
     for bits in (1, 2, 3, 4):
-        for n in (1, 15, 31, 33, 257, 20_001):
+        for n in (1, 15, 31, 33, 257, 20_001, 150_001):
             codes, packed, norms, cen, R = data(d, bits, n, n)
             out = ops().dequantize_mse_packed(packed, norms.to(dt), cen, R, bits, d)
             check(out, codes, norms.to(dt).float(), cen, R, dt)
@@ -74,6 +75,30 @@ def test_cache_and_new_tokens(d, vb, dt):
         if T:
             check(k[:, :, :T], kc.view(B, H, T, d), kno[:, :, :T].float(), kcen, kR, dt)
             check(v[:, :, :T], vc.view(B, H, T, d), vno[:, :, :T].float(), vcen, vR, dt)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d,vb", [(64, 2), (64, 3), (64, 4), (128, 2), (128, 3), (128, 4)])
+def test_cache_of_many_tokens(d, vb, dt):
+    """More 32-token steps than the launch has waves: each takes one after another, its next codes
+    on their way."""
+    from turboquant_kv import ops
+    from turboquant_kv._lib import ops as tops
+    B, H, T, cap = 8, 8, 2100, 2112
+    g = torch.Generator(device=DEV).manual_seed(d + vb)
+    kc, kp_rows, kn, kcen, kR = data(d, 4, B * H * T, 1)
+    vc, vp_rows, vn, vcen, vR = data(d, vb, B * H * T, 2)
+    kp = torch.zeros(B, H, cap, d // 2, device=DEV, dtype=torch.uint8)
+    vp = torch.zeros(B, H, cap // 64, 8 * vb * d, device=DEV, dtype=torch.uint8)
+    ops.pack_decode_layout(kp_rows.view(B * H, T, -1), kp.view(B * H, cap, -1), d, 4, False, 0)
+    ops.pack_decode_layout(vp_rows.view(B * H, T, -1), vp.view(B * H, cap // 64, -1), d, vb, True, 0)
+    kno, vno = (torch.full((B, H, cap), float("nan"), device=DEV, dtype=dt) for _ in range(2))
+    kno[:, :, :T], vno[:, :, :T] = kn.view(B, H, T).to(dt), vn.view(B, H, T).to(dt)
+    x = torch.randn(B, H, 3, d, generator=g, device=DEV).to(dt)
+    k, v = tops().dequantize_cache_dl(kp, kno, vp, vno, T, kcen, kR, vcen, vR, dt, x, x * 2)
+    assert torch.equal(k[:, :, T:], x) and torch.equal(v[:, :, T:], x * 2)
+    check(k[:, :, :T], kc.view(B, H, T, d), kno[:, :, :T].float(), kcen, kR, dt)
+    check(v[:, :, :T], vc.view(B, H, T, d), vno[:, :, :T].float(), vcen, vR, dt)
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])

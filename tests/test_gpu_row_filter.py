@@ -91,6 +91,19 @@ def test_equals_exact_scan(d):
     assert hit >= 40
 
 
+@pytest.mark.parametrize("d,bits,prod,N", [(200, 4, 1, 300_007), (100, 3, 0, 300_007), (128, 4, 0, 300_007),
+                                           (16, 2, 0, 1_100_003), (37, 3, 1, 1_100_003), (64, 4, 1, 1_100_003)])
+def test_several_groups_per_wave(d, bits, prod, N):
+    """Row counts at which a wave takes one group after another, its next rows on their way, and
+    the sample is spread over the table (its stride above 1; two groups a bucket above 1,048,576)."""
+    db = random_rows(N, d, bits, prod, d)
+    db["p"][5000:5040] = db["p"][7].clone()  # ties
+    db["nm"][5000:5040] = db["nm"][7].clone()
+    g = torch.Generator(device=DEV).manual_seed(d)
+    for Q, k in ((17, 10), (5, 100)):
+        assert same(db, torch.randn(Q, d, generator=g, device=DEV).half(), k, unflagged=True)
+
+
 def test_rounds_of_queries():
     """More queries than one round of lists holds."""
     db = database(9000, 100, 3, 0, 0, 1)
