@@ -52,7 +52,7 @@ struct RfArgs {
   float* buckets;        // [passes 16][nbk]
   float* tau;            // [passes 16]
   int nbk, per_bucket, sstride, nsgroups, nb;
-  bool fine;             // a bucket per 16 rows (per_bucket 1), else per_bucket groups
+  bool wide;             // rot and qjl are read 16 bytes at a time
   int* cnt;              // [passes][nb][16]
   float* chi;            // [passes][nb][16][kRfCap]
   float* clo;
@@ -76,7 +76,7 @@ __global__ __launch_bounds__(PROD ? 512 : 256) void rf_query_kernel(RfArgs a) {
   const int qi = blockIdx.x, mi = threadIdx.x >> 8, j = threadIdx.x & 255, d = a.d;
   const bool real = qi < a.nq;
   const float* __restrict__ mat = mi ? a.qjl : a.rot;
-  const bool wide = (d & 3) == 0 && (reinterpret_cast<uintptr_t>(mat) & 15u) == 0;
+  const bool wide = a.wide;
   const int nch = real ? (d + C - 1) / C : 0;  // uniform
   // thread j's pieces of a chunk: row r = 16 i + j / 16, columns 4 (j % 16) ..
   struct Chunk {
@@ -362,7 +362,8 @@ __device__ __forceinline__ void rf_bounds(const RfQuery<KT, PROD>& q, int r, flo
   bound = __builtin_fmaf(fabsf(n), b, 0x1p-100f);
 }
 
-template <int BITS, int KT, bool PROD, bool PAIRS>
+// FINE: a bucket per 16 rows (per_bucket 1), else per per_bucket groups.
+template <int BITS, int KT, bool PROD, bool PAIRS, bool FINE>
 __global__ __launch_bounds__(kRfThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void rf_sample_kernel(RfArgs a) {
 #pragma clang fp contract(off)
   __shared__ __attribute__((aligned(16))) RfTables t;
@@ -384,7 +385,7 @@ __global__ __launch_bounds__(kRfThreads) __attribute__((amdgpu_waves_per_eu(2, 2
     for (int r = 0; r < 4; ++r) {
       const float v = row_max16(bmax[r]);
       if ((lane & 15) == 0) a.buckets[(size_t)(tile * kRfQ + 4 * (lane >> 4) + r) * a.nbk + at] = v;
-      bmax[r] = -INFINITY;
+      if (FINE) bmax[r] = -INFINITY;
     }
   };
   for (int u = 0; u < a.per_bucket; ++u) {
@@ -407,10 +408,10 @@ __global__ __launch_bounds__(kRfThreads) __attribute__((amdgpu_waves_per_eu(2, 2
         const float lo = mid - b;  // no bound from an overflowed one
         if (valid && lo < INFINITY) bmax[r] = fmaxf(bmax[r], lo);
       }
-      if (a.fine) store(4 * bucket + rt);  // uniform
+      if (FINE) store(4 * bucket + rt);
     }
   }
-  if (!a.fine && bucket < a.nbk) store(bucket);
+  if (!FINE && bucket < a.nbk) store(bucket);
 }
 
 // One block per query: tau = its k-th largest bucket maximum, by bits of an order-preserving key

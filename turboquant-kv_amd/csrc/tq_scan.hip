@@ -3895,8 +3895,9 @@ int launch_rf_t(const RfArgs& a, const RfLayout& L, hipStream_t st) {
   const int waves = (L.nsgroups + L.per_bucket - 1) / L.per_bucket;
   hipLaunchKernelGGL((rf_query_kernel<KT, PROD>), dim3(passes * kRfQ), dim3(PROD ? 512 : 256), 0, st, a);
   TQ_LAUNCH_CHECK("rf_query_kernel");
-  hipLaunchKernelGGL((rf_sample_kernel<BITS, KT, PROD, PAIRS>), dim3((unsigned)((waves + kRfWaves - 1) / kRfWaves), passes),
-                     dim3(kRfThreads), 0, st, a);
+  const dim3 sample((unsigned)((waves + kRfWaves - 1) / kRfWaves), passes);
+  if (L.fine) hipLaunchKernelGGL((rf_sample_kernel<BITS, KT, PROD, PAIRS, true>), sample, dim3(kRfThreads), 0, st, a);
+  else hipLaunchKernelGGL((rf_sample_kernel<BITS, KT, PROD, PAIRS, false>), sample, dim3(kRfThreads), 0, st, a);
   TQ_LAUNCH_CHECK("rf_sample_kernel");
   hipLaunchKernelGGL(rf_tau_kernel, dim3(passes * kRfQ), dim3(kRfThreads), 0, st, a);
   TQ_LAUNCH_CHECK("rf_tau_kernel");
@@ -3953,7 +3954,8 @@ int launch_rf(const ScanArgs& s0, int bits, bool pairs, char* ws, const RfLayout
     a.clo = reinterpret_cast<float*>(ws + L.clo);
     a.cid = reinterpret_cast<int*>(ws + L.cid);
     a.nbk = L.nbk; a.per_bucket = L.per_bucket; a.sstride = L.sstride; a.nsgroups = L.nsgroups; a.nb = L.nb;
-    a.fine = L.fine;
+    a.wide = (s.d & 3) == 0 &&
+             ((reinterpret_cast<uintptr_t>(s.rot) | (s.signs ? reinterpret_cast<uintptr_t>(s.qjl) : 0)) & 15u) == 0;
     a.out_s = s.out_s; a.out_i = s.out_i;
     int rc;
     if (s.signs) rc = bits == 2 ? launch_rf_bits<2, true>(a, L, pairs, st) : launch_rf_bits<3, true>(a, L, pairs, st);
