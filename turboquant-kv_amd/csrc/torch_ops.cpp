@@ -1340,8 +1340,8 @@ void cache_append_dl(const at::Tensor& key, const at::Tensor& value, at::Tensor&
   }
 }
 
-// The first T tokens of a decode-layout cache dequantized to `out_like`'s dtype, then the new
-// tokens key_new / value_new [B, H, s, d] as they are: (keys, values) [B, H, T + s, d].
+// The first T tokens of a decode-layout cache dequantized to `dtype`, then the new tokens key_new /
+// value_new [B, H, s, d] converted to it: (keys, values) [B, H, T + s, d].
 std::tuple<at::Tensor, at::Tensor> dequantize_cache_dl(
     const at::Tensor& kp, const at::Tensor& kn, const at::Tensor& vp, const at::Tensor& vn, int64_t T,
     const at::Tensor& kcentroids, const at::Tensor& krotation, const at::Tensor& vcentroids,

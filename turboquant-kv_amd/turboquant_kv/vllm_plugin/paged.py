@@ -178,8 +178,8 @@ class PagedKVPools:
         if "kp" in st and key.dtype == value.dtype and key.dtype in (torch.bfloat16, torch.float16):
             # quantized and stored by one launch
             shape = (n, H, self.head_dim)
-            _ops().paged_write_dl(key.reshape(shape), value.reshape(shape), sm, st["kp"], st["kn"], st["vt"], st["vn"], self.R_k, self.kbnd,
-                                  self.R_v, self.vbnd)
+            _ops().paged_write_dl(key.reshape(shape), value.reshape(shape), sm, st["kp"], st["kn"],
+                                  st["vt"], st["vn"], self.R_k, self.kbnd, self.R_v, self.vbnd)
             return
         kq = self._quantize(key.to(self.device), self.R_k, self.kbnd, self.kcen,
                             getattr(self, "S_k", None), self.config.key_bits)
