@@ -147,7 +147,10 @@ def test_few_results_around_a_million_rows_scan_exactly(d, bits, N, nq, k):
     base = lambda n, q, kk: L.tq_scan_workspace_bytes(q, d, bits, n, kk)  # noqa: E731
     assert size(N, nq, k) == base(N, nq, k)
     assert size(N, nq, 32) > base(N, nq, 32) and size(N // 10, nq, k) > base(N // 10, nq, k)
+    for n, kk, on in ((12_000, 1, False), (12_000, 10, False), (12_000, 32, True), (100_000, 1, True)):
+        assert (size(n, 700, kk) > base(n, 700, kk)) == on, (n, kk)  # many queries over few rows
     if d == 64 and bits == 4:  # prod pair rows
+        assert size(12_000, 700, 10, 1, 1) == base(12_000, 700, 10)
         assert size(10_000_000, 2, 10, 1, 1) == base(10_000_000, 2, 10)
         assert size(10_000_000, 3, 10, 1, 1) == base(10_000_000, 3, 10)
         assert size(10_000_000, 2, 100, 1, 1) > base(10_000_000, 2, 100)

@@ -3871,17 +3871,25 @@ RfLayout rf_layout(int64_t nq, int d, int64_t N, int k, bool prod, size_t base) 
 //     -> 188, k = 64 196 -> 199, k = 128 533 -> 208) and three a few million rows at most (3M 92
 //     -> 83, 10M 171 -> 189).  k = 33 .. 64: 64 dims 1M rows, 3 queries 52 -> 61, 4 queries 70 -> 61;
 //     128 dims 300,000, 4 queries 53 -> 56, 6 queries 78 -> 57
+//   hundreds of queries over few rows of 64 / 128 dims, where the filter's lists and merge, per
+//     query, cost more than the rows: 4-bit planes, 700 queries, 64 dims 8,192 rows k = 1 67 -> 129,
+//     k = 10 93 -> 131, 40,000 rows k = 10 299 -> 208; 128 dims 8,192 rows k = 10 123 -> 170, 20,000
+//     269 -> 233; prod pair rows of 64 dims, 3 bits, 12,000 rows, k = 10 93 -> 144
 bool rf_applies(int64_t nq, int d, int64_t N, int k, int bits, bool prod, bool pairs) {
   if (nq < 1 || nq > INT_MAX || N < 8192 || bits < 2 || bits > (prod ? 3 : 4) || d < 16) return false;
   const int bpp = (d + 7) / 8;
+  const bool many = nq > kRfRound;
   if (pairs) {
     if (!prod || nq < 2) return false;
+    if (many && d == 64 && k <= 64 && N < (k <= 16 ? 24000 : 16000)) return false;
+    if (many && d == 128 && k <= (bits == 3 ? 40 : 16) && N < 16000) return false;
     if (d == 64 && nq == 2 && k <= 64) return false;
     if (d == 64 && nq == 3 && k < kSmallK && N > 5000000) return false;
     return (double)N * nq * d >= (k <= kSmallK ? 4e8 : k <= 64 && nq <= 5 ? 2e8 : 1.2e8);
   }
   if (bpp != 8 && bpp != 16) return true;
   if (k > kSmallK) return nq >= 2;
+  if (many && k <= 16 && N < (k <= 2 ? 2 : 1) * (bpp == 8 ? 24000 : 16000)) return false;
   if (k <= 4 && N > 250000 && N < 2000000) {
     if (k <= 2 && bits == 4 && bpp == 8) return nq >= 7;
     if (nq == 4 && (bits == 4 || (k <= 2 && bpp == 8))) return N <= 500000;
