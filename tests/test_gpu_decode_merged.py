@@ -35,3 +35,21 @@ def test_merged_equals_decode_then_merge(d, vb, B, hkv, G, tc, norm, dt, kv_dt):
         got = ops().decode_attention_dl_merged(*args, k1, v1)
         assert got.dtype == want.dtype and torch.equal(got, want)
         assert torch.equal(got[0], v1[0].repeat_interleave(G, 0).to(dt))  # no history: its own value
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_merge_rounds_the_new_value_then_the_sum(d):
+    """o e^(lse - m) + v e^(s - m) is rounded as one fma over the rounded second product: with s = 20
+    above lse the weights are e^-20 (read back from o = 1, v = 0) and 1, their sum 1."""
+    from turboquant_kv._lib import ops
+    g = torch.Generator(device=DEV).manual_seed(d)
+    q, k = torch.zeros(2, 8, d, device=DEV), torch.zeros(2, 2, d, device=DEV)
+    q[..., 0], k[..., 0] = 4.0, 5.0
+    lse = torch.zeros(2, 8, device=DEV)
+    w = ops().decode_merge_token(torch.ones_like(q), lse, q, k, torch.zeros_like(k), 1.0)
+    assert torch.equal(w, w[0, 0, 0].expand_as(w)) and abs(float(w[0, 0, 0]) / 2.0611536e-09 - 1) < 1e-6
+    o = torch.randn(2, 8, d, generator=g, device=DEV) * 4e8
+    v = torch.randn(2, 2, d, generator=g, device=DEV)
+    got = ops().decode_merge_token(o, lse, q, k, v, 1.0)
+    want = (o.double() * w.double() + v.repeat_interleave(4, 1).double()).float()  # 48-bit product: exact
+    assert torch.equal(got, want)

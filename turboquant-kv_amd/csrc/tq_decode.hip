@@ -473,8 +473,8 @@ __device__ __forceinline__ float merge_new_token(float dot, float scale, float o
   const float sn = dot * scale;
   const float m = fmaxf(lh, sn);
   const float wh = expf(lh - m), wn = expf(sn - m), den = wh + wn;
-  const float x = round_to(o, q_dt) * wh + v * wn;
-  return x / den;
+  // the fma written out: each caller's compilation rounds the same way
+  return fmaf(round_to(o, q_dt), wh, v * wn) / den;
 }
 
 // One D-thread block per query row (D = head_dim, 64 or 128): log-sum-exp merge of the
