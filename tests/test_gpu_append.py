@@ -132,3 +132,24 @@ def paged_write_equals_separate_ops(slots, block, vb, dt, H, nb, tab, g, name):
     tops().paged_write_dl(k, v, slots, kp, kn, vt, vn, Rk, bk, Rv, bv)
     for got, w, what in zip((kp, kn, vt, vn), want, ("keys", "key norms", "values", "value norms")):
         assert torch.equal(got, w), (what, name)
+
+
+def test_cache_append_tracked_and_empty():
+    """Keys or values with a gradient mark the cache and what is computed from it (a backward says
+    that there is none); an append of no tokens is refused in every layout."""
+    from turboquant_kv import QuantizedKVCache, TurboQuantConfig
+    g = torch.Generator(device=DEV).manual_seed(5)
+    k, v = (torch.randn(1, 2, 40, 64, generator=g, device=DEV).bfloat16() for _ in range(2))
+    q = torch.randn(1, 4, 64, generator=g, device=DEV).bfloat16()
+    make = lambda kb=4: QuantizedKVCache(TurboQuantConfig(key_bits=kb, value_bits=3), 1, 128, 2, 64)  # noqa: E731
+    plain, tracked = make(), make()
+    plain.append(0, k, v)
+    tracked.append(0, k.clone().requires_grad_(), v)
+    for a, b in zip((plain._kstore, plain._vstore, plain._key_norms, plain._val_norms),
+                    (tracked._kstore, tracked._vstore, tracked._key_norms, tracked._val_norms)):
+        assert torch.equal(a[0], b[0])
+    assert not plain.decode_attention(0, q).requires_grad
+    assert tracked.decode_attention(0, q).requires_grad
+    for kb in (4, 3):
+        with pytest.raises(RuntimeError):
+            make(kb).append(0, k[:, :, :0], v[:, :, :0])

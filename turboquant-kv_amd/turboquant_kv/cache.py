@@ -167,7 +167,8 @@ class QuantizedKVCache:
             self._val_fp[layer_id][:, :, sl] = value.half()
             self.seq_lens[layer_id] += s
             return
-        if self._dl:  # K and V quantized, packed and stored by one op
+        grad = torch.is_grad_enabled() and (key.requires_grad or value.requires_grad)
+        if self._dl and s > 0 and not grad:  # K and V quantized, packed and stored by one op
             _ops().cache_append_dl(key, value, self._kstore[layer_id], self._key_norms[layer_id],
                                    self._vstore[layer_id], self._val_norms[layer_id], pos, self._key_rotation,
                                    self._kbnd, self._val_rotation, self._vbnd, self._kbits_stored,
@@ -193,8 +194,14 @@ class QuantizedKVCache:
     def _store(self, layer_id: int, values: bool, rows: torch.Tensor, pos: int) -> None:
         """Write bit-plane rows [B*H, s, P] at tokens pos..pos+s of every (batch, head)."""
         st = (self._vstore if values else self._kstore)[layer_id]
+        B, H = self.batch_size, self.num_heads
         s = rows.shape[1]
-        st[:, :, pos:pos + s] = rows.view(self.batch_size, self.num_heads, s, -1)
+        if self._dl:
+            bits = self._vbits_stored if values else self._kbits_stored
+            ops.pack_decode_layout(rows, st.view(B * H, st.shape[2], st.shape[3]), self.head_dim,
+                                   bits, values, pos)
+        else:
+            st[:, :, pos:pos + s] = rows.view(B, H, s, -1)
 
     def _ops_quantize(self, x, R, bnd, cen, S, bits):
         flat = x.reshape(-1, self.head_dim)
