@@ -40,3 +40,28 @@ def test_forward_prefill_rows(dtype, how):
     if out is not None:
         assert got.data_ptr() == out.data_ptr()
     assert got.dtype == dtype and torch.equal(got, want)  # the same sums, converted once
+
+
+def test_forward_keeps_graph_and_strides():
+    """Through queries with a gradient a prefill's result is a node of the graph (whose backward says
+    that there is none); a decode step's result has the strides of dense queries in another order."""
+    from turboquant_kv.vllm_plugin import PagedKVPools, TurboQuantAttentionMetadata
+    pools = PagedKVPools(TurboQuantConfig(), 1, 4, 16, 2, 64, DEV, layout="decode")
+    g = torch.Generator(device=DEV).manual_seed(3)
+    q, k, v = (torch.randn(20, h, 64, generator=g, device=DEV).bfloat16() for h in (4, 2, 2))
+    table = torch.arange(4, device=DEV, dtype=torch.int32).view(1, 4)
+
+    def step(query, n, t, npf):
+        md = TurboQuantAttentionMetadata(
+            num_prefills=npf, slot_mapping=torch.arange(t - n, t, device=DEV), block_tables=table,
+            seq_lens=torch.tensor([t], dtype=torch.int32, device=DEV),
+            query_start_loc=torch.tensor([0, n], dtype=torch.int32, device=DEV))
+        return pools.forward(query, k[:n], v[:n], md, 0.125)
+
+    plain = step(q, 20, 20, 1)
+    tracked = step(q.clone().requires_grad_(), 20, 20, 1)
+    assert tracked.requires_grad and not plain.requires_grad and torch.equal(plain, tracked.detach())
+    one = q[:1]
+    other = one.transpose(1, 2).contiguous().transpose(1, 2)
+    a, b = step(one, 1, 21, 0), step(other, 1, 21, 0)
+    assert torch.equal(a, b) and b.stride() == other.stride() != a.stride()

@@ -331,7 +331,8 @@ class PagedKVPools:
         layer = md.layer_id
         self.write(layer, key, value, md.slot_mapping)
         npf = md.num_prefills
-        if npf == 0 and output is None and 0 < query.shape[0] == md.block_tables.shape[0]:
+        if (npf == 0 and output is None and 0 < query.shape[0] == md.block_tables.shape[0]
+                and query.is_contiguous()):
             # decode tokens only: the kernel's own output is the result
             return self.decode(layer, query, md.block_tables, md.seq_lens.to(self.device, torch.int32),
                                scale).to(query)
@@ -346,8 +347,11 @@ class PagedKVPools:
                                   md.seq_lens[:npf].to(torch.int64)]).tolist()
                 qsl, lens = both[:npf + 1], both[npf + 1:]
             # a result that shares the queries' memory takes a sequence's rows after they are read
-            # (float64 queries are computed in float32, so their result is converted)
+            # (float64 queries are computed in float32, so their result is converted; through
+            # queries with a gradient the result is a node of the graph)
             direct = (out.dtype == query.dtype and query.dtype != torch.float64
+                      and query.dim() == 3 and out.shape[1:] == query.shape[1:]
+                      and not (query.requires_grad and torch.is_grad_enabled())
                       and out.device == query.device == self.kcen.device
                       and out.untyped_storage().data_ptr() != query.untyped_storage().data_ptr())
             for i in range(npf):
