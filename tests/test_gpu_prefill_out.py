@@ -65,3 +65,21 @@ def test_forward_keeps_graph_and_strides():
     other = one.transpose(1, 2).contiguous().transpose(1, 2)
     a, b = step(one, 1, 21, 0), step(other, 1, 21, 0)
     assert torch.equal(a, b) and b.stride() == other.stride() != a.stride()
+
+
+def test_forward_under_vmap():
+    """A prefill and a decode step mapped over batches of queries."""
+    from turboquant_kv.vllm_plugin import PagedKVPools, TurboQuantAttentionMetadata
+    pools = PagedKVPools(TurboQuantConfig(), 1, 4, 16, 2, 64, DEV, layout="decode")
+    g = torch.Generator(device=DEV).manual_seed(3)
+    q, k, v = (torch.randn(2, 20, h, 64, generator=g, device=DEV).bfloat16() for h in (4, 2, 2))
+    for n, t, npf in ((20, 20, 1), (1, 21, 0)):
+        md = TurboQuantAttentionMetadata(
+            num_prefills=npf, slot_mapping=torch.arange(t - n, t, device=DEV),
+            block_tables=torch.arange(4, device=DEV, dtype=torch.int32).view(1, 4),
+            seq_lens=torch.tensor([t], dtype=torch.int32, device=DEV),
+            query_start_loc=torch.tensor([0, n], dtype=torch.int32, device=DEV),
+            query_start_loc_cpu=[0, n], seq_lens_cpu=[t])
+        step = lambda x: pools.forward(x, k[0, :n], v[0, :n], md, 0.125)  # noqa: E731
+        want = torch.stack([step(q[0, :n]), step(q[1, :n])])
+        assert torch.equal(torch.vmap(step)(q[:, :n]), want)

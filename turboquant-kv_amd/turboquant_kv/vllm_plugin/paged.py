@@ -67,6 +67,14 @@ class TurboQuantAttentionMetadata:
     seq_lens_cpu: Optional[List[int]] = None
 
 
+def _shares_memory(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Whether they lie in one storage, or cannot say (the tensors of a vmap have none)."""
+    try:
+        return a.untyped_storage().data_ptr() == b.untyped_storage().data_ptr()
+    except NotImplementedError:
+        return True
+
+
 def gather_value_tiles(vt_pool: torch.Tensor, block_table: torch.Tensor, T: int) -> torch.Tensor:
     """Value tiles of tokens 0..T-1 of one sequence from a decode-layout pool, in the
     contiguous decode layout [H, ceil(T/64), 512 vb] (unpack_decode_layout's input)."""
@@ -353,7 +361,7 @@ class PagedKVPools:
                       and query.dim() == 3 and out.shape[1:] == query.shape[1:]
                       and not (query.requires_grad and torch.is_grad_enabled())
                       and out.device == query.device == self.kcen.device
-                      and out.untyped_storage().data_ptr() != query.untyped_storage().data_ptr())
+                      and not _shares_memory(out, query))
             for i in range(npf):
                 a, b = qsl[i], qsl[i + 1]
                 if b <= a:
